@@ -40,7 +40,8 @@ struct pfchem_ctx {
   LaunchCfg vlaunch[2][kBuckets];
   int32_t* buckets = nullptr;  // kBuckets lists of ncell entries, then the counts
   int64_t bucket_cap = 0;
-  int32_t* esc_list = nullptr;  // cells the one-lane pass handed over, then their count
+  int32_t* esc_list = nullptr;  // the number of cells the one-lane pass handed over (64 bits,
+                                // kEscHeader ints), then the cells
   int64_t esc_cap = 0;
   // steps that use the scratch lists held here (escalated cells, status
   // scratch, size buckets) are ordered on the device: each records this
@@ -146,10 +147,10 @@ void* static_scratch_ptr(int device) {
 // stream the earlier launch used.
 const int kStateRing = 256;
 constexpr size_t kCursorWords = 1024;  // 8 KiB of cursors per descriptor slot
-// handed-over cells above which the FP64 one-lane kernel runs before the
-// team pass (the team pass alone takes a short list faster: its time is one
-// cell's latency)
+// handed-over cells of a small network above which the FP64 one-lane kernel
+// runs before the team pass
 constexpr int kLaneListMin = 4096;
+constexpr int kEscHeader = 64;         // ints before the hand-over list: its count
 
 unsigned long long* slot_cursors(pfchem_ctx* ctx, int k) {
   return ctx->counter + (size_t)k * kCursorWords;
@@ -421,6 +422,7 @@ int pfchem_create(const pfchem_network* net, const pfchem_options* opt, int devi
     ctx->max_lds = lds;
   // MI355X / MI300-class parts have 32 CUs per XCD
   ctx->nxcd = ctx->num_cus >= 64 && ctx->num_cus % 32 == 0 ? ctx->num_cus / 32 : 1;
+  if (ctx->nxcd > 21) ctx->nxcd = 21;  // three sets of cursors fit a descriptor slot
 
   const int nc = net->neqcplx, nm = net->nkinmnrl;
   Packer P;
@@ -945,8 +947,8 @@ static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double d
                       .blocks_per_cu;
   hipError_t e = hipSuccess;
   a.rescue = 0;
-  // the rescue pass walks only the cells the one-lane pass handed over
-  // (listed by a compaction kernel; larger grids walk all cells)
+  // the rescue pass walks only the cells the one-lane pass handed over,
+  // which that pass lists (larger grids walk all cells)
   DevState dr = d;
   dr.status = st;
   const bool listed = ncell <= 0x7fffffff;
@@ -956,12 +958,14 @@ static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double d
       if (ctx->esc_list) (void)hipFree(ctx->esc_list);
       ctx->esc_list = nullptr;
       ctx->esc_cap = 0;
-      if (hipMalloc(&ctx->esc_list, sizeof(int32_t) * ((size_t)ncell + 64)) != hipSuccess)
+      if (hipMalloc(&ctx->esc_list, sizeof(int32_t) * ((size_t)ncell + kEscHeader)) != hipSuccess)
         return fail(ctx, PFCHEM_ERR_NOMEM, "escalated-cell list");
       ctx->esc_cap = ncell;
     }
-    dr.cell_list = ctx->esc_list;
-    dr.list_count = ctx->esc_list + ncell;
+    a.esc_count = (unsigned long long*)ctx->esc_list;
+    a.esc_list = ctx->esc_list + kEscHeader;
+    dr.cell_list = a.esc_list;
+    dr.list_count = ctx->esc_list;  // the low word of the count (< 2^31)
   }
   // one descriptor slot (and its cursors) for both launches of this step
   int k = 0;
@@ -972,33 +976,34 @@ static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double d
   e = scratch_order(ctx, s);
   if (e == hipSuccess && ctx->pass_timing) e = hipEventRecord(ctx->pass_t0, s);
   if (e == hipSuccess)
-    e = lane_launch(ctx->lane_src, ctx->device, mixed ? 1 : 0, a, ctx->num_cus, bpc, cursors, s);
+    e = lane_launch(ctx->lane_src, ctx->device, mixed ? 1 : 0, a, ctx->num_cus, bpc, cursors,
+                    3 * ctx->nxcd, s);
   if (e == hipSuccess && ctx->pass_timing) {
     e = hipEventRecord(ctx->pass_t1, s);
     if (e == hipSuccess) ctx->pass_recorded = true;
   }
   if (e != hipSuccess)
     return hip_fail(ctx, e, mixed ? "lane kernel launch (FP32)" : "lane kernel launch (FP64)");
-  if (listed) {
-    e = launch_escalated_list(st, ncell, ctx->esc_list, ctx->esc_list + ncell, s);
-    if (e != hipSuccess) return hip_fail(ctx, e, "escalated-cell list");
-    if (mixed) {
-      // a long list goes through the FP64 one-lane kernel first (per cell
-      // several times cheaper than a team, at a longer latency for its
-      // slowest cell); the team pass takes what that pass hands over.  A
-      // short list (the kernel reads its length) is left to the team pass.
-      LaneArgs b = a;
-      b.rescue = 1;
-      b.list = ctx->esc_list;
-      b.list_count = ctx->esc_list + ncell;
-      b.list_min = kLaneListMin;
-      e = lane_launch(ctx->lane_src, ctx->device, 0, b, ctx->num_cus,
-                      ctx->launch[PFCHEM_KERNEL_BATCHED_FP64].blocks_per_cu, cursors, s);
-      if (e != hipSuccess) return hip_fail(ctx, e, "lane kernel launch (FP64 list)");
-    }
+  if (listed && mixed) {
+    // the FP64 one-lane kernel takes the handed-over cells first (it returns
+    // at once for an empty list), the team pass what that kernel hands over:
+    // a Newton iteration of the team kernel, which reads the network's
+    // tables from memory, takes 35 us, the one-lane kernel's 10 us.  A small
+    // network's short list is left to the team pass, which is as fast there.
+    LaneArgs b = a;
+    b.rescue = 1;
+    b.list = a.esc_list;
+    b.list_count = ctx->esc_list;
+    b.esc_list = nullptr;
+    b.list_min = ctx->net.naqcomp < kProdMinAq ? kLaneListMin : 0;
+    e = lane_launch(ctx->lane_src, ctx->device, 0, b, ctx->num_cus,
+                    ctx->launch[PFCHEM_KERNEL_BATCHED_FP64].blocks_per_cu, cursors + 16 * ctx->nxcd,
+                    0, s);
+    if (e != hipSuccess) return hip_fail(ctx, e, "lane kernel launch (FP64 list)");
   }
   e = launch_team_step(ctx->dnet, ctx->dnet_dev, slot, ncell, dt, kTeamRescue64,
-                       ctx->team_default, cursors, ctx->num_cus, ctx->nxcd, s, true);
+                       ctx->team_default, cursors + 32 * ctx->nxcd, ctx->num_cus, ctx->nxcd, s,
+                       true);
   if (e == hipSuccess) e = release_slot(ctx, k, s);
   if (e == hipSuccess) e = scratch_release(ctx, s);
   if (e != hipSuccess) return hip_fail(ctx, e, "team rescue launch");

@@ -77,7 +77,8 @@ int team_supports(const DevNet& n, const LaunchCfg& cfg, bool mixed);
 // dn / ds: device copies of the network / state descriptors.  mixed = 0:
 // FP64; 1: the FP32 pass and then an FP64 pass over the cells the FP32
 // pass could not converge (needs the per-cell status array); kTeamRescue64:
-// only the FP64 pass over cells whose status is kTeamEscalate.
+// only the FP64 pass over cells whose status is kTeamEscalate (cursors
+// cleared by the caller).
 constexpr int kTeamRescue64 = 2;
 constexpr int kTeamEscalate = 16;
 hipError_t launch_team_step(const DevNet& n, const DevNet* dn, const DevState* ds,
@@ -90,10 +91,6 @@ hipError_t launch_team_step(const DevNet& n, const DevNet* dn, const DevState* d
 // counts are cleared by a fill kernel on `stream` first.
 constexpr int kBuckets = 3;
 constexpr int kBucketBound[kBuckets] = {16, 32, 64};
-// the cells whose status is kTeamEscalate into list[0 .. *count) (any
-// order); ncell < 2^31
-hipError_t launch_escalated_list(const int32_t* status, int64_t ncell, int32_t* list,
-                                 int32_t* count, hipStream_t stream);
 hipError_t launch_buckets(const int32_t* nact, int64_t ncell, int naq, int32_t* lists,
                           int32_t* counts, hipStream_t stream);
 

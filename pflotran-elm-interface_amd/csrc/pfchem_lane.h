@@ -47,8 +47,10 @@ struct LaneArgs {
   int list_min;
   const int* list;
   const int* list_count;
+  int* esc_list;
+  unsigned long long* esc_count;
 };
-static_assert(sizeof(LaneArgs) == 208, "LaneArgs layout");
+static_assert(sizeof(LaneArgs) == 224, "LaneArgs layout");
 
 // adjoint kernel arguments; the same layout as pflane::SensArgs
 struct LaneSensArgs {
@@ -82,6 +84,10 @@ constexpr int kLaneSensSub = 8;  // sub-steps the adjoint kernel records per cel
 // first line of an adjoint module's source (followed by lane_source)
 constexpr char kLaneAdjointDefine[] = "#define PFLANE_ADJOINT 1\n";
 
+// networks of at least this many primaries evaluate mass action as products
+// of powers (pfchem_lane.hpp)
+constexpr int kProdMinAq = 9;
+
 // 1 if the lane kernel handles this network and these options (else `why`)
 int lane_supported(const pfchem_network* net, const pfchem_options* opt, std::string& why);
 // full device source: the network as constants followed by the template
@@ -92,12 +98,12 @@ int lane_compile(const std::string& src, int device, std::string& err);
 int lane_compile_only(const std::string& src, std::vector<char>* code, std::string& err);
 // launch the FP32 (f32 = 1) or FP64 kernel of a compiled source over
 // args.ncell cells; persistent grid of num_cus x min(blocks_per_cu,
-// occupancy) workgroups of 256 lanes (blocks_per_cu <= 0: occupancy)
+// occupancy) workgroups of 256 lanes (blocks_per_cu <= 0: occupancy).  With
+// nclear > 0 one fill kernel first clears that many cursors (the passes of a
+// step use consecutive sets of nxcd) and *args.esc_count.
 hipError_t lane_launch(const std::string& src, int device, int f32, const LaneArgs& args,
-                       int num_cus, int blocks_per_cu, unsigned long long* cursors,
+                       int num_cus, int blocks_per_cu, unsigned long long* cursors, int nclear,
                        hipStream_t stream);
-// resident 256-lane workgroups per CU of a compiled kernel (0: not compiled)
-int lane_occupancy(const std::string& src, int device, int f32);
 // launch the adjoint kernel of a compiled source, one cell per lane
 hipError_t lane_adjoint_launch(const std::string& src, int device, const LaneSensArgs& args,
                                hipStream_t stream);

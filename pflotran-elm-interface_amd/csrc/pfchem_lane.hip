@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hiprtc.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -104,6 +105,36 @@ void rows(const int32_t* ids, const double* st, int n, int ms, std::vector<int>&
   }
 }
 
+// Reaction rows the kernel evaluates as products of powers: integer
+// stoichiometry of at most 4, at most 32 factors in all, and a constant log K
+// without a water-activity factor.  km 2^ke = exp(-log K ln 10), the
+// exponent formed as the log form does.
+struct ProdRows {
+  std::vector<int> on, ke;
+  std::vector<double> km;
+};
+ProdRows prod_rows(const std::vector<std::vector<double>>& nu, const double* logK,
+                   const double* h2o, int naq, const pfchem_options* opt, bool has_coef) {
+  ProdRows p;
+  for (size_t k = 0; k < nu.size(); ++k) {
+    bool ok = naq >= kProdMinAq && (opt->isothermal || !has_coef) && !(opt->use_activity_h2o && h2o && h2o[k] != 0.0);
+    int sum = 0;
+    for (double v : nu[k]) {
+      const int iv = (int)v;
+      ok = ok && (double)iv == v && iv != 0 && std::abs(iv) <= 4;
+      sum += std::abs(iv);
+    }
+    const double lnk = logK ? -logK[k] * 2.30258509299 : 0.0;
+    ok = ok && sum <= 32 && std::fabs(lnk) < 10000.0;
+    int e = 0;
+    long double m = ok ? std::frexp(std::exp((long double)lnk), &e) : 0.0L;
+    p.on.push_back(ok ? 1 : 0);
+    p.km.push_back((double)m);
+    p.ke.push_back(e);
+  }
+  return p;
+}
+
 struct Module {
   hipModule_t mod = nullptr;
   hipFunction_t f32 = nullptr, f64 = nullptr, adj = nullptr;
@@ -112,8 +143,9 @@ struct Module {
 std::mutex g_mu;
 std::map<std::pair<int, std::string>, Module> g_mods;  // (device, source) -> module
 
-__global__ void lane_zero_cursors(unsigned long long* c, int n) {
+__global__ void lane_zero_cursors(unsigned long long* c, int n, unsigned long long* count) {
   if ((int)threadIdx.x < n) c[16 * threadIdx.x] = 0ull;
+  if (threadIdx.x == 0 && count) *count = 0ull;
 }
 
 }  // namespace
@@ -280,6 +312,34 @@ std::string lane_source(const pfchem_network* net, const pfchem_options* opt) {
   if (net->kinmnrl_irreversible)
     for (int m = 0; m < nm; ++m) irr[m] = net->kinmnrl_irreversible[m];
   g.ivec("MNRL_IRREV", irr);
+  // mass action: product or log form per row; what each primary needs
+  // (NEED_PROD 1: mantissa and exponent, 2: the reciprocal mantissa too)
+  {
+    const ProdRows cp = prod_rows(cnu, net->eqcplx_logK, net->eqcplxh2ostoich, naq, opt,
+                                  net->eqcplx_logKcoef != nullptr);
+    const ProdRows mp = prod_rows(mnu, net->kinmnrl_logK, net->kinmnrlh2ostoich, naq, opt,
+                                  net->kinmnrl_logKcoef != nullptr);
+    std::vector<int> need(naq, 0), ln(naq, 0);
+    auto scan = [&](const ProdRows& p, const std::vector<std::vector<int>>& id,
+                    const std::vector<std::vector<double>>& nu) {
+      for (size_t k = 0; k < id.size(); ++k)
+        for (size_t q = 0; q < id[k].size(); ++q) {
+          if (!p.on[k]) ln[id[k][q]] = 1;
+          else need[id[k][q]] = std::max(need[id[k][q]], nu[k][q] < 0.0 ? 2 : 1);
+        }
+    };
+    scan(cp, cid, cnu);
+    scan(mp, mid, mnu);
+    g.ivec("CPLX_PROD", cp.on);
+    g.dvec("CPLX_KM", cp.km);
+    g.ivec("CPLX_KE", cp.ke);
+    g.ivec("MNRL_PROD", mp.on);
+    g.dvec("MNRL_KM", mp.km);
+    g.ivec("MNRL_KE", mp.ke);
+    g.i("ANY_PROD", *std::max_element(need.begin(), need.end()) > 0 ? 1 : 0);
+    g.ivec("NEED_PROD", need);
+    g.ivec("NEED_LN", ln);
+  }
   // immobile decay
   std::vector<int> did;
   std::vector<double> dk;
@@ -353,7 +413,7 @@ int lane_compile_only(const std::string& src, std::vector<char>* code, std::stri
 }
 
 hipError_t lane_launch(const std::string& src, int device, int f32, const LaneArgs& args,
-                       int num_cus, int blocks_per_cu, unsigned long long* cursors,
+                       int num_cus, int blocks_per_cu, unsigned long long* cursors, int nclear,
                        hipStream_t stream) {
   Module m;
   {
@@ -370,9 +430,11 @@ hipError_t lane_launch(const std::string& src, int device, int f32, const LaneAr
   if (blocks > max_blocks) blocks = max_blocks;
   if (blocks > args.nxcd) blocks -= blocks % args.nxcd;
   if (blocks < 1) blocks = 1;
-  lane_zero_cursors<<<1, 64, 0, stream>>>(cursors, args.nxcd);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (nclear > 0) {
+    lane_zero_cursors<<<1, 64, 0, stream>>>(cursors, nclear, args.esc_count);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   LaneArgs a = args;
   a.cursors = cursors;
   void* params[] = {&a};
@@ -395,13 +457,6 @@ hipError_t lane_adjoint_launch(const std::string& src, int device, const LaneSen
   void* params[] = {&a};
   return hipModuleLaunchKernel(m.adj, (unsigned)blocks, 1, 1, 256, 1, 1, 0, stream, params,
                                nullptr);
-}
-
-int lane_occupancy(const std::string& src, int device, int f32) {
-  std::lock_guard<std::mutex> lk(g_mu);
-  auto it = g_mods.find(std::make_pair(device, src));
-  if (it == g_mods.end()) return 0;
-  return f32 ? it->second.blocks_per_cu32 : it->second.blocks_per_cu64;
 }
 
 }  // namespace pfchem

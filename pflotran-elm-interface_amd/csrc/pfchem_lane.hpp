@@ -21,19 +21,24 @@
 //   * in the log formulation the aqueous Jacobian of RReact is
 //       J_log = jc (diag(x) + S^T diag(m) S) + sum_m g_m nu_m nu_m^T,
 //     jc = phi s 1000 V rho/1000 / dt, with g_m = dIm/dQK QK V rho/1000 >= 0
-//     for every TST rate law: symmetric positive definite.  It is scaled
-//     symmetrically to unit diagonal, A = D^-1/2 M D^-1/2 (M = J_log / jc),
-//     and factored as L D L^T without pivoting; the linear formulation solves
+//     for every TST rate law: symmetric positive definite.  M = J_log / jc is
+//     factored as L D L^T without pivoting; the linear formulation solves
 //     the same system and multiplies the step by x (J_lin = J_log diag(x)^-1);
 //   * immobile rows are diagonal (accumulation + first-order decay);
 //   * JT = float: the off-diagonal entries are accumulated pre-scaled by
 //     1/sqrt(x_i x_j) in FP32 (|entry| <= sqrt(D_i D_j / x_i x_j)), scaled to
-//     A in FP32 and factored in FP32; the diagonal, totals, residual, log K
-//     sums, exponentials, the update and every convergence test stay FP64
-//     (the Newton iteration is the iterative refinement);
+//     unit diagonal in FP32 and factored in FP32; the diagonal, totals,
+//     residual, log K sums, exponentials, the update and every convergence
+//     test stay FP64 (the Newton iteration is the iterative refinement);
 //   * a pivot below the tolerance, a non-finite entry, or (FP32) a Newton
 //     iteration that does not converge hands the cell, with its inputs
 //     untouched, to a later pass: status kEscalate.
+// With packed FP32 off, FP32 and FP64 instructions issue at the same rate on
+// gfx950, and forming an FP32 entry takes three instructions (multiply,
+// convert, FMA) where an FP64 one takes an FMA: the FP32 pass saves registers
+// only.  Where the FP32 Newton iteration ends is decided by the rounding of
+// its factorization in one cell of a hundred, so its arithmetic is left as it
+// is rather than moved to FP64 accumulation or another scaling.
 #pragma once
 
 namespace pflane {
@@ -46,6 +51,10 @@ constexpr double kIdealGas = 8.31446;
 constexpr double kRtMinSat = 1.0e-40;
 constexpr int kEscalate = 16;        // per-cell status: handed to the next pass
 constexpr int kClaim = 64;           // cells per refill of a wave's queue
+// Waiting lanes that make a wave write back and load.  1,048,576 cells of
+// the 15-primary network, 7 iterations a cell: 4.4 ms at 1, 3.7 at 16, 3.6 at
+// 24 and 32 (the waiting lanes idle); uneven 262,144 cells 3.6, 3.1, 3.1 ms.
+constexpr int kServe = 24;
 enum : int { kOk = 0, kMaxIter = 1, kSingular = 2 };
 enum : int { kFreqNewtonIter = 2 };
 
@@ -78,8 +87,10 @@ struct Args {
   int list_min;  // with a list: the pass does nothing unless it holds more cells
   const int* list;        // NULL, or the cells to step: list[0 .. *list_count)
   const int* list_count;  // device memory, written by an earlier kernel
+  int* esc_list;                  // NULL, or receives the cells handed over,
+  unsigned long long* esc_count;  // in any order, and their number
 };
-static_assert(sizeof(Args) == 208, "Args layout");
+static_assert(sizeof(Args) == 224, "Args layout");
 
 template <int V>
 struct IC {
@@ -98,11 +109,56 @@ __host__ __device__ constexpr int tri(int i, int j) {
   return i > j ? i * (i - 1) / 2 + j : j * (j - 1) / 2 + i;
 }
 
+// A copy of a wave-uniform value that the compiler cannot trace to its
+// source: row offsets k * ld derived from it are formed where they are used
+// instead of being hoisted out of the persistent loop, where 450 of them
+// were spilled to vector lanes and read back in every iteration.
+__device__ __forceinline__ i64 opaque(i64 v) {
+#ifdef __AMDGCN__
+  asm volatile("" : "+s"(v));
+#endif
+  return v;
+}
+
+// keeps the loads written before it ahead of the uses written after it
+__device__ __forceinline__ void issue_loads() {
+#ifdef __AMDGCN__
+  __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
 // FP64 exp / log (inlined: out-of-line calls cost more than the
 // instruction-cache misses of the larger unrolled loop, measured on MI355X)
 __device__ __forceinline__ double pf_exp(double v) { return exp(v); }
 __device__ __forceinline__ double pf_log(double v) { return log(v); }
 
+// exp(v) for |v| <= 600: v = n ln 2 + r with |r| <= ln 2 / 2, the Taylor series of
+// exp(r) to r^13 (remainder below 5e-18) and one ldexp; without the range
+// tests of exp, which the clipped Newton step does not need
+__device__ __forceinline__ double exp_bounded(double v) {
+  const double n = __builtin_rint(v * 1.4426950408889634074);
+  double r = fma(-n, 0x1.62e42fefa3800p-1, v);  // ln 2 in two parts, the first
+  r = fma(-n, 0x1.ef35793c76730p-45, r);        // short enough for n * part to be exact
+  double p = 1.0 / 6227020800.0;
+  p = fma(p, r, 1.0 / 479001600.0);
+  p = fma(p, r, 1.0 / 39916800.0);
+  p = fma(p, r, 1.0 / 3628800.0);
+  p = fma(p, r, 1.0 / 362880.0);
+  p = fma(p, r, 1.0 / 40320.0);
+  p = fma(p, r, 1.0 / 5040.0);
+  p = fma(p, r, 1.0 / 720.0);
+  p = fma(p, r, 1.0 / 120.0);
+  p = fma(p, r, 1.0 / 24.0);
+  p = fma(p, r, 1.0 / 6.0);
+  p = fma(p, r, 0.5);
+  p = fma(p, r, 1.0);
+  p = fma(p, r, 1.0);
+  return __builtin_ldexp(p, (int)n);
+}
+__device__ __forceinline__ double exp_step(double v) {
+  if constexpr (Net::ANY_PROD && Net::MAX_DLNC <= 600.0) return exp_bounded(v);
+  else return pf_exp(v);
+}
 // 1/g by the hardware reciprocal estimate refined with two Newton-Raphson
 // steps r <- r + r (1 - g r) (within about one ulp of the quotient; g > 0,
 // normal)
@@ -142,6 +198,118 @@ __device__ __forceinline__ double mnrl_lnk(double lnT, double tk) {
     return -interp_logk(Net::MNRL_COEF[M], lnT, tk) * kLogToLn;
 }
 
+// Mass action as products of powers.  With integer stoichiometry and a
+// constant log K, K prod a^nu is formed from the activities' mantissas
+// (in [1/2, 1), their reciprocals for negative nu) with the exponents summed
+// as integers and applied once by ldexp, so no intermediate leaves the FP64
+// range whatever the activities.  One multiplication per unit of |nu| (six
+// for an average complex of the 15-primary network) replaces the exponential
+// of each complex and the logarithm of each primary, which were 40 % of the
+// step kernel's instructions; a product of at most 32 factors is good to
+// ~1e-14, the exponential of a sum of logarithms of size 40 to the same.
+// Networks of up to 8 primaries keep the log form and the arithmetic that
+// goes with it (exp_step, the factorization's scaling): with 8 primaries and
+// 32 complexes a cell in a hundred meets the 1e-14 residual test, and one in
+// ten thousand the iteration limit, by rounding alone, so other rounding
+// would move its sub-steps; their kernels are short either way.
+// Rows with other stoichiometry, log K(T) or a water-activity factor keep the
+// log form (Net::CPLX_PROD / MNRL_PROD).
+template <int NA1>
+struct Acts {
+  double m[NA1], r[NA1];  // mantissa of the activity and its reciprocal
+  int e[NA1];             // exponent
+  double l[NA1];          // ln activity (rows in log form)
+};
+// ln gamma (networks without product rows) or gamma, as the kernels keep it
+__device__ __forceinline__ double act_keep(double gamma) {
+  if constexpr (Net::ANY_PROD) return gamma;
+  else return pf_log(gamma);
+}
+// activity of primary I at molality x; a <= 0 (or NaN) gives NaN, as its
+// logarithm would
+template <int I, int NA1>
+__device__ __forceinline__ void act_set(Acts<NA1>& A, double x, double kept) {
+  if constexpr (!Net::ANY_PROD) {
+    A.l[I] = pf_log(x) + kept;
+    return;
+  }
+  const double a = x * kept;
+  if constexpr (Net::NEED_PROD[I] != 0) {
+    const double v = a > 0.0 ? a : __builtin_nan("");
+    int e = 0;
+    A.m[I] = __builtin_frexp(v, &e);
+    A.e[I] = e;
+    if constexpr (Net::NEED_PROD[I] > 1) A.r[I] = rcp_nr(A.m[I]);
+  }
+  if constexpr (Net::NEED_LN[I] != 0) A.l[I] = pf_log(a);
+}
+template <int P>
+__device__ __forceinline__ double ipow(double b) {
+  if constexpr (P == 1) return b;
+  else if constexpr (P == 2) return b * b;
+  else if constexpr (P == 3) return b * b * b;
+  else return (b * b) * (b * b);
+}
+// scale K_k prod a^nu of complex K as p 2^e
+template <int K, int NA1>
+__device__ __forceinline__ double cplx_pe(const Acts<NA1>& A, double lnT, double tk, double ln_aw,
+                                          double scale, int& e) {
+  if constexpr (Net::CPLX_PROD[K] != 0) {
+    double p = Net::CPLX_KM[K] * scale;
+    e = Net::CPLX_KE[K];
+    sfor<0, Net::CPLX_N[K]>([&](auto Q) {
+      constexpr int i = Net::CPLX_ID[K][decltype(Q)::value];
+      constexpr int nu = (int)Net::CPLX_NU[K][decltype(Q)::value];
+      if constexpr (nu > 0) p *= ipow<nu>(A.m[i]);
+      else p *= ipow<-nu>(A.r[i]);
+      e += nu * A.e[i];
+    });
+    return p;
+  } else {
+    e = 0;
+    double lnQK = cplx_lnk<K>(lnT, tk);
+    if constexpr (Net::CPLX_H2O[K] != 0.0) lnQK += Net::CPLX_H2O[K] * ln_aw;
+    sfor<0, Net::CPLX_N[K]>([&](auto Q) {
+      constexpr int a = decltype(Q)::value;
+      lnQK += Net::CPLX_NU[K][a] * A.l[Net::CPLX_ID[K][a]];
+    });
+    return pf_exp(lnQK) * scale;
+  }
+}
+template <int K, int NA1>
+__device__ __forceinline__ double cplx_q(const Acts<NA1>& A, double lnT, double tk, double ln_aw,
+                                         double scale) {
+  int e;
+  const double p = cplx_pe<K>(A, lnT, tk, ln_aw, scale, e);
+  if constexpr (Net::CPLX_PROD[K] != 0) return __builtin_ldexp(p, e);
+  else return p;
+}
+// Q/K of kinetic mineral M
+template <int M, int NA1>
+__device__ __forceinline__ double mnrl_q(const Acts<NA1>& A, double lnT, double tk,
+                                         double ln_aw) {
+  if constexpr (Net::MNRL_PROD[M] != 0) {
+    double p = Net::MNRL_KM[M];
+    int e = Net::MNRL_KE[M];
+    sfor<0, Net::MNRL_N[M]>([&](auto Q) {
+      constexpr int i = Net::MNRL_ID[M][decltype(Q)::value];
+      constexpr int nu = (int)Net::MNRL_NU[M][decltype(Q)::value];
+      if constexpr (nu > 0) p *= ipow<nu>(A.m[i]);
+      else p *= ipow<-nu>(A.r[i]);
+      e += nu * A.e[i];
+    });
+    return __builtin_ldexp(p, e);
+  } else {
+    double lnQK = mnrl_lnk<M>(lnT, tk);
+    if constexpr (Net::MNRL_H2O[M] != 0.0) lnQK += Net::MNRL_H2O[M] * ln_aw;
+    sfor<0, Net::MNRL_N[M]>([&](auto Q) {
+      constexpr int a = decltype(Q)::value;
+      lnQK += Net::MNRL_NU[M][a] * A.l[Net::MNRL_ID[M][a]];
+    });
+    return pf_exp(lnQK);
+  }
+}
+
 // RKineticMineral rate of mineral M (reaction_mineral.F90:729-908): Im per
 // unit bulk volume and dIm/dQK per unit volume; active = the reference does
 // not `cycle` past the mineral
@@ -150,8 +318,7 @@ struct MRate {
   bool active;
 };
 template <int M>
-__device__ __forceinline__ MRate mineral_rate(double lnQK, double QK, double vf, double area,
-                                              double temp) {
+__device__ __forceinline__ MRate mineral_rate(double QK, double vf, double area, double temp) {
   MRate r{0.0, 0.0, false};
   constexpr bool temkin = Net::HAS_TEMKIN, mscale = Net::HAS_MINSCALE;
   double sig = 1.0;
@@ -195,22 +362,44 @@ __device__ __forceinline__ MRate mineral_rate(double lnQK, double QK, double vf,
   return r;
 }
 
+// secondary molality of complex K: with coefficients fixed during the step
+// gi holds the inverse of each (Z^2, a0) class's; otherwise g receives the
+// Debye-Hueckel coefficient at the ionic strength I
+template <int K, bool NEWTON_ACT, int NA1, int NG1>
+__device__ __forceinline__ double cplx_m(const Acts<NA1>& act, double lnT, double tk, double ln_aw,
+                                         const double (&gi)[NG1], double sI, double I, double& g) {
+  if constexpr (NEWTON_ACT) {
+    g = 1.0;
+    if constexpr (Net::CPLX_Z[K] > 1.0e-10 || Net::CPLX_Z[K] < -1.0e-10)
+      g = dh_gamma(Net::CPLX_Z[K], Net::CPLX_A0[K], sI, I);
+    return cplx_q<K>(act, lnT, tk, ln_aw, 1.0) / g;
+  } else if constexpr (Net::CPLX_GCLS[K] >= 0) {
+    return cplx_q<K>(act, lnT, tk, ln_aw, gi[Net::CPLX_GCLS[K]]);
+  } else {
+    return cplx_q<K>(act, lnT, tk, ln_aw, 1.0);
+  }
+}
+
+__device__ __forceinline__ void hand_over(const Args& A, i64 c) {
+  A.status[c] = kEscalate;
+  if (A.esc_list) A.esc_list[atomicAdd(A.esc_count, 1ull)] = (int)c;
+}
+
 // One reaction step for cells [0, ncell) (or, with rescue, the cells whose
-// status is kEscalate).  JT: precision of the off-diagonal Jacobian entries
-// and of the factorization.
+// status is kEscalate).  JT: precision of the factorization.
 template <typename JT>
 __device__ __forceinline__ void lane_step(const Args& A) {
   constexpr int NAQ = Net::NAQ, NIMM = Net::NIMM, N = NAQ + NIMM, NC = Net::NC, NM = Net::NM;
   constexpr int NA1 = NAQ > 0 ? NAQ : 1, NM1 = NM > 0 ? NM : 1;
   constexpr int NT = NAQ > 1 ? NAQ * (NAQ - 1) / 2 : 1;
-  constexpr bool F32 = sizeof(JT) == 4;
   constexpr bool NEWTON_ACT = Net::ACT_FREQ == kFreqNewtonIter && NAQ > 0;
   // per-class inverse activity coefficients of the complexes (activity
   // coefficients fixed during the step)
   constexpr int NG = NEWTON_ACT ? 0 : Net::NGCLS;
   constexpr int NG1 = NG > 0 ? NG : 1;
   constexpr int kLdsFields = 2 * N + NAQ + 3 * NM + NG > 0 ? 2 * N + NAQ + 3 * NM + NG : 1;
-  // pivot tolerance of the unit-diagonal factorization
+  constexpr bool F32 = sizeof(JT) == 4;
+  // pivot tolerance of the factorization, relative to the diagonal
   constexpr double kPivTol = F32 ? 1.0e-6 : 1.0e-13;
   const i64 ld = A.ld;
   const int lane = (int)__lane_id();
@@ -233,7 +422,7 @@ __device__ __forceinline__ void lane_step(const Args& A) {
   const int tid = (int)threadIdx.x;
 #define PF_GUESS(i) lsm[(0 + (i)) * 256 + tid]
 #define PF_TINIT(i) lsm[(N + (i)) * 256 + tid]
-#define PF_LNGAM(i) lsm[(2 * N + (i)) * 256 + tid]
+#define PF_GAM(i) lsm[(2 * N + (i)) * 256 + tid]
 #define PF_VF(m) lsm[(2 * N + NAQ + (m)) * 256 + tid]
 #define PF_AREA(m) lsm[(2 * N + NAQ + NM + (m)) * 256 + tid]
 #define PF_RLAST(m) lsm[(2 * N + NAQ + 2 * NM + (m)) * 256 + tid]
@@ -255,6 +444,99 @@ __device__ __forceinline__ void lane_step(const Args& A) {
   for (int i = 0; i < N; ++i) x[i] = 1.0;
 
   for (;;) {
+    // lanes without work wait until kServe of them do (or none iterates):
+    // writing back and loading touch some 230 rows of the state for however
+    // few lanes
+    const unsigned long long waiting = __ballot(mode == 2 || (cell < 0 && !exhausted));
+    const bool serve = __popcll(waiting) >= kServe || !__ballot(mode == 1);
+    if (serve) {
+    // ---------------- write finished cells back ----------------
+    // totals, secondary molalities, rates and the last sub-step's kinetic
+    // update at the final unknowns; apart from the Newton evaluation, which
+    // then carries no stores and no write-out tests
+    if (mode == 2) {
+      const i64 c = cell;
+      const i64 lo = opaque(ld);
+      const bool ok = status == 0;
+      double I = 0.0, sI = 0.0;
+      if constexpr (NEWTON_ACT) {  // the last iteration's ionic strength
+        I = I_last;
+        sI = sqrt(I);
+      }
+      Acts<NA1> act;
+      double tot[NA1];
+      sfor<0, NAQ>([&](auto Q) {
+        constexpr int i = decltype(Q)::value;
+        act_set<i>(act, x[i], PF_GAM(i));
+        tot[i] = 0.0;
+      });
+      double gi[NG1];
+      sfor<0, NG>([&](auto Q) {
+        constexpr int q = decltype(Q)::value;
+        gi[q] = PF_GINV(q);
+      });
+      double* ps = A.sec_molal + c;
+      double* pg = A.sec_act_coef + c;
+      sfor<0, NC>([&](auto K) {
+        constexpr int k = decltype(K)::value;
+        double g = 1.0;
+        const double m = cplx_m<k, NEWTON_ACT>(act, lnT, tk, ln_aw, gi, sI, I, g);
+        *ps = m;
+        ps += lo;
+        if constexpr (NEWTON_ACT) {
+          *pg = g;
+          pg += lo;
+        }
+        sfor<0, Net::CPLX_N[k]>([&](auto Q) {
+          constexpr int a = decltype(Q)::value;
+          tot[Net::CPLX_ID[k][a]] += Net::CPLX_NU[k][a] * m;
+        });
+      });
+      double* pp = A.pri_molal + c;
+      double* pt = A.total + c;
+      double* pa = A.pri_act_coef + c;
+      sfor<0, NAQ>([&](auto Q) {
+        constexpr int i = decltype(Q)::value;
+        *pp = x[i];
+        const bool keep = ok && ((small >> i) & 1u);  // original value restored
+        if (!keep) *pt = (!ok && restore) ? PF_TINIT(i) : (x[i] + tot[i]) * dkl;
+        if constexpr (NEWTON_ACT) *pa = Net::ANY_PROD ? PF_GAM(i) : pf_exp(PF_GAM(i));
+        pp += lo;
+        pt += lo;
+        pa += lo;
+      });
+      sfor<0, NIMM>([&](auto Q) {
+        constexpr int i = NAQ + decltype(Q)::value;
+        const bool keep = ok && ((small >> i) & 1u);
+        if (!keep) A.immobile[(i - NAQ) * lo + c] = (!ok && restore) ? PF_TINIT(i) : x[i];
+      });
+      sfor<0, NM>([&](auto M) {
+        constexpr int m = decltype(M)::value;
+        if (kin) {
+          // RUpdateKineticState of the last sub-step (reaction_mineral.F90:
+          // 1456-1525): rates at the final state, volume fractions of the
+          // sub-step's start
+          double r = 0.0;
+          const double ar = PF_AREA(m);
+          if (ar != 0.0) r = mineral_rate<m>(mnrl_q<m>(act, lnT, tk, ln_aw), PF_VF(m), ar, temp).Im;
+          double v = PF_VF(m) + r * Net::MNRL_VM[m] * tdt;
+          if (v < 0.0) v = 0.0;
+          PF_VF(m) = v;
+          PF_RLAST(m) = r;
+        }
+        A.mnrl_volfrac[m * lo + c] = PF_VF(m);
+        if (A.mnrl_rate) A.mnrl_rate[m * lo + c] = PF_RLAST(m);
+      });
+      if constexpr (NEWTON_ACT && Net::ACT_H2O) {
+        if (A.ln_act_h2o) A.ln_act_h2o[c] = ln_aw;
+      }
+      if (A.num_iterations) A.num_iterations[c] = nit_total;
+      if (A.num_sub_steps) A.num_sub_steps[c] = nsub;
+      if (A.status) A.status[c] = status;
+      cell = -1;
+      mode = 0;
+    }
+
     // ---------------- work stealing: hand out cells ----------------
     {
       bool needy = cell < 0 && !exhausted;
@@ -297,38 +579,71 @@ __device__ __forceinline__ void lane_step(const Args& A) {
       }
     }
     if (__all(cell < 0)) break;  // every lane of the wave is done
+    }
     if (cell < 0) continue;
     const i64 c = cell;
 
     // ---------------- load the cell; RStep set-up ----------------
+    if (mode == 2) continue;  // waits to be written back
     if (mode == 0) {
+      const i64 lo = opaque(ld);
+      // every load of a block is issued before the first value is used: one
+      // wavefront per SIMD has nothing else to hide a load's latency with
       por = A.porosity[c];
       sat = A.saturation[c];
       const double den = A.den_kg[c];
       vol = A.volume[c];
       temp = A.temperature ? A.temperature[c] : 25.0;
+      ln_aw = (Net::ACT_H2O && A.ln_act_h2o) ? A.ln_act_h2o[c] : 0.0;
+      double tin[N], gam[NA1], vf[NM1], ar[NM1];
+      {
+        const double* pp = A.pri_molal + c;
+        const double* pt = A.total + c;
+        const double* pg = A.pri_act_coef + c;
+        sfor<0, NAQ>([&](auto I) {
+          constexpr int i = decltype(I)::value;
+          x[i] = *pp;
+          tin[i] = *pt;
+          gam[i] = *pg;
+          pp += lo;
+          pt += lo;
+          pg += lo;
+        });
+        sfor<0, NIMM>([&](auto I) {
+          constexpr int i = decltype(I)::value;
+          x[NAQ + i] = A.immobile[i * lo + c];
+          tin[NAQ + i] = x[NAQ + i];
+        });
+        const double* pv = A.mnrl_volfrac + c;
+        const double* pa = A.mnrl_area + c;
+        sfor<0, NM>([&](auto M) {
+          constexpr int m = decltype(M)::value;
+          vf[m] = *pv;
+          ar[m] = *pa;
+          pv += lo;
+          pa += lo;
+        });
+      }
+      issue_loads();
       tk = temp + 273.15;
       lnT = pf_log(tk);
-      ln_aw = (Net::ACT_H2O && A.ln_act_h2o) ? A.ln_act_h2o[c] : 0.0;
       dkl = den * 1.0e-3;
       psv = por * sat * 1000.0 * vol;
-      double tin[N];
       sfor<0, NAQ>([&](auto I) {
         constexpr int i = decltype(I)::value;
-        x[i] = A.pri_molal[i * ld + c];
-        tin[i] = A.total[i * ld + c];
-        PF_LNGAM(i) = pf_log(A.pri_act_coef[i * ld + c]);
+        PF_GAM(i) = act_keep(gam[i]);
       });
-      sfor<0, NIMM>([&](auto I) {
-        constexpr int i = decltype(I)::value;
-        x[NAQ + i] = A.immobile[i * ld + c];
-        tin[NAQ + i] = x[NAQ + i];
+      sfor<0, NM>([&](auto M) {
+        constexpr int m = decltype(M)::value;
+        PF_VF(m) = vf[m];
+        PF_AREA(m) = ar[m];
+        PF_RLAST(m) = 0.0;
       });
       if constexpr (NEWTON_ACT) {
         sec_I = sec_sum = 0.0;
         sfor<0, NC>([&](auto K) {
           constexpr int k = decltype(K)::value;
-          const double mk = A.sec_molal[k * ld + c];
+          const double mk = A.sec_molal[k * lo + c];
           sec_I += mk * Net::CPLX_Z[k] * Net::CPLX_Z[k];
           sec_sum += mk;
         });
@@ -339,38 +654,42 @@ __device__ __forceinline__ void lane_step(const Args& A) {
         // each (Z^2, a0) class keeps one inverse coefficient for the whole
         // step.  A cell whose input coefficients break that structure is
         // handed to the team kernel, which reads them per complex.
-        bool cons = true;
+        bool odd = false;
         double g0[NG1];
-        sfor<0, NC>([&](auto K) {
-          constexpr int k = decltype(K)::value;
-          constexpr int q = Net::CPLX_GCLS[k];
-          const double g = A.sec_act_coef[k * ld + c];
-          if constexpr (q < 0) {
-            cons = cons && g == 1.0;
-          } else if constexpr (Net::CPLX_GFIRST[k]) {
-            g0[q] = g;
-            PF_GINV(q) = rcp_nr(g);
-          } else {
-            cons = cons && g == g0[q];
-          }
+        const double* pg = A.sec_act_coef + c;
+        constexpr int CH = 16;  // complexes per block of loads
+        sfor<0, (NC + CH - 1) / CH>([&](auto B) {
+          constexpr int k0 = decltype(B)::value * CH, k1 = k0 + CH < NC ? k0 + CH : NC;
+          double g[CH];
+          sfor<k0, k1>([&](auto K) {
+            g[decltype(K)::value - k0] = *pg;
+            pg += lo;
+          });
+          issue_loads();
+          sfor<k0, k1>([&](auto K) {
+            constexpr int k = decltype(K)::value;
+            constexpr int q = Net::CPLX_GCLS[k];
+            if constexpr (q < 0) {
+              odd |= !(g[k - k0] == 1.0);
+            } else if constexpr (Net::CPLX_GFIRST[k]) {
+              g0[q] = g[k - k0];
+              PF_GINV(q) = rcp_nr(g[k - k0]);
+            } else {
+              odd |= !(g[k - k0] == g0[q]);
+            }
+          });
         });
-        if (!cons && A.escalate) {
-          A.status[c] = kEscalate;
+        if (odd && A.escalate) {
+          hand_over(A, c);
           cell = -1;
           continue;
         }
       }
-      sfor<0, NM>([&](auto M) {
-        constexpr int m = decltype(M)::value;
-        PF_VF(m) = A.mnrl_volfrac[m * ld + c];
-        PF_AREA(m) = A.mnrl_area[m * ld + c];
-        PF_RLAST(m) = 0.0;
-      });
       if constexpr (!Net::FULL_GEOCHEM) {
         // RStep early exit (reaction.F90:3601-3605)
         sfor<0, NAQ>([&](auto I) {
           constexpr int i = decltype(I)::value;
-          A.pri_molal[i * ld + c] = tin[i] / den * 1.0e3;
+          A.pri_molal[i * lo + c] = tin[i] / den * 1.0e3;
         });
         if (A.num_iterations) A.num_iterations[c] = 0;
         if (A.num_sub_steps) A.num_sub_steps[c] = 0;
@@ -411,8 +730,8 @@ __device__ __forceinline__ void lane_step(const Args& A) {
         r0 = 0.0;
       }
     }
-    const bool iterate = mode == 1;
-    if (iterate) ++nit;
+    if (mode == 2) continue;  // no call left: written back next time round
+    ++nit;
 
     // ---------------- RTotal + RReaction at x ----------------
     const bool wet = !(sat < kRtMinSat);
@@ -421,11 +740,10 @@ __device__ __forceinline__ void lane_step(const Args& A) {
     const double jc = psvd * dkl;
     const double wm = wet ? 1.0 : 0.0;
     // activity coefficients per Newton iteration (LAG at the current pri
-    // and last secondary molalities); the write-out evaluation reuses the
-    // ionic strength of the last iteration
+    // and last secondary molalities)
     double I = 0.0, sI = 0.0;
     if constexpr (NEWTON_ACT) {
-      if (iterate) {
+      {
         double Ip = 0.0, sp = 0.0;
         sfor<0, NAQ>([&](auto Q) {
           constexpr int i = decltype(Q)::value;
@@ -437,25 +755,23 @@ __device__ __forceinline__ void lane_step(const Args& A) {
         sfor<0, NAQ>([&](auto Q) {
           constexpr int i = decltype(Q)::value;
           if constexpr (Net::ZP[i] > 1.0e-10 || Net::ZP[i] < -1.0e-10)
-            PF_LNGAM(i) = pf_log(dh_gamma(Net::ZP[i], Net::A0P[i], sI, I));
+            PF_GAM(i) = act_keep(dh_gamma(Net::ZP[i], Net::A0P[i], sI, I));
           else
-            PF_LNGAM(i) = 0.0;
+            PF_GAM(i) = act_keep(1.0);
         });
         if constexpr (Net::ACT_H2O) {
           const double a = 1.0 - 0.017 * (sp + sec_sum);
           ln_aw = a > 0.0 ? pf_log(a) : 0.0;
         }
         I_last = I;
-      } else {
-        I = I_last;
-        sI = sqrt(I);
       }
     }
-    double lnact[NA1], sig[NA1], tot[NA1], D[NA1];
+    Acts<NA1> act;
+    double tot[NA1], D[NA1], sig[NA1];
     JT S[NT];
     sfor<0, NAQ>([&](auto Q) {
       constexpr int i = decltype(Q)::value;
-      lnact[i] = pf_log(x[i]) + PF_LNGAM(i);
+      act_set<i>(act, x[i], PF_GAM(i));
       // FP32 entries are accumulated pre-scaled by sig_i sig_j (any scale
       // works: it is divided out exactly below); FP64 ones are not scaled
       sig[i] = F32 ? __builtin_amdgcn_rsq(x[i]) : 1.0;
@@ -464,7 +780,6 @@ __device__ __forceinline__ void lane_step(const Args& A) {
     });
 #pragma unroll
     for (int q = 0; q < NT; ++q) S[q] = (JT)0;
-    const bool wout = mode == 2;
     double nsI = 0.0, nss = 0.0;
     double gi[NG1];
     sfor<0, NG>([&](auto Q) {
@@ -475,27 +790,8 @@ __device__ __forceinline__ void lane_step(const Args& A) {
     sfor<0, NC>([&](auto K) {
       constexpr int k = decltype(K)::value;
       constexpr int ns = Net::CPLX_N[k];
-      double lnQK = cplx_lnk<k>(lnT, tk);
-      if constexpr (Net::CPLX_H2O[k] != 0.0) lnQK += Net::CPLX_H2O[k] * ln_aw;
-      sfor<0, ns>([&](auto Q) {
-        constexpr int a = decltype(Q)::value;
-        lnQK += Net::CPLX_NU[k][a] * lnact[Net::CPLX_ID[k][a]];
-      });
-      double m;
-      double g = 1.0;
-      if constexpr (NEWTON_ACT) {
-        if constexpr (Net::CPLX_Z[k] > 1.0e-10 || Net::CPLX_Z[k] < -1.0e-10)
-          g = dh_gamma(Net::CPLX_Z[k], Net::CPLX_A0[k], sI, I);
-        m = pf_exp(lnQK) / g;
-      } else if constexpr (Net::CPLX_GCLS[k] >= 0) {
-        m = pf_exp(lnQK) * gi[Net::CPLX_GCLS[k]];
-      } else {
-        m = pf_exp(lnQK);
-      }
-      if (wout) {
-        A.sec_molal[k * ld + c] = m;
-        if constexpr (NEWTON_ACT) A.sec_act_coef[k * ld + c] = g;
-      }
+      double g;
+      const double m = cplx_m<k, NEWTON_ACT>(act, lnT, tk, ln_aw, gi, sI, I, g);
       if constexpr (NEWTON_ACT) {
         nsI += m * (Net::CPLX_Z[k] * Net::CPLX_Z[k]);
         nss += m;
@@ -546,18 +842,27 @@ __device__ __forceinline__ void lane_step(const Args& A) {
     sfor<0, NM>([&](auto Mi) {
       constexpr int mi = decltype(Mi)::value;
       constexpr int ns = Net::MNRL_N[mi];
-      double lnQK = mnrl_lnk<mi>(lnT, tk);
-      if constexpr (Net::MNRL_H2O[mi] != 0.0) lnQK += Net::MNRL_H2O[mi] * ln_aw;
-      sfor<0, ns>([&](auto Q) {
-        constexpr int a = decltype(Q)::value;
-        lnQK += Net::MNRL_NU[mi][a] * lnact[Net::MNRL_ID[mi][a]];
-      });
       rt[mi] = 0.0;
       const double ar = PF_AREA(mi);
-      if (ar != 0.0) {  // zero area gives Im = 0
-        const double QK = pf_exp(lnQK);
-        const MRate r = mineral_rate<mi>(lnQK, QK, PF_VF(mi), ar, temp);
-        if (r.active) {
+      // zero area gives Im = 0.  The plain rate law runs without branches:
+      // with a few minerals active per cell some lane of a wavefront has
+      // each of them, and the branches kept the complexes' arithmetic from
+      // being scheduled across them
+      constexpr bool plain = Net::HAS_TEMKIN + Net::HAS_MINSCALE + Net::HAS_AFFPOWER +
+                                 Net::HAS_LIMITER + Net::HAS_IRREV + Net::HAS_THRESHOLD +
+                                 Net::HAS_EA == 0;
+      if (plain || ar != 0.0) {
+        const double QK = mnrl_q<mi>(act, lnT, tk, ln_aw);
+        MRate r;
+        if constexpr (plain) {
+          const double aff = 1.0 - QK;
+          r.active = ar != 0.0 && (PF_VF(mi) > 0.0 || QK > 1.0);
+          r.Im = r.active ? -(ar * aff) * Net::MNRL_K[mi] : 0.0;
+          r.dIm = r.active ? ar * Net::MNRL_K[mi] : 0.0;
+        } else {
+          r = mineral_rate<mi>(QK, PF_VF(mi), ar, temp);
+        }
+        if (plain || r.active) {
           rt[mi] = r.Im;
           // dry cells: RReaction adds nothing (reaction.F90:4083)
           const double Rm = r.Im * vol * wm;
@@ -590,49 +895,6 @@ __device__ __forceinline__ void lane_step(const Args& A) {
       nr2 += res[i] * res[i];
     }
 
-    if (wout) {
-      // ---------------- write the cell back ----------------
-      const bool ok = status == 0;
-      if (kin) {
-        // RUpdateKineticState of the last sub-step (reaction_mineral.F90:
-        // 1456-1525): rates at the final state, volume fractions of the
-        // sub-step's start
-        sfor<0, NM>([&](auto M) {
-          constexpr int m = decltype(M)::value;
-          double v = PF_VF(m) + rt[m] * Net::MNRL_VM[m] * tdt;
-          if (v < 0.0) v = 0.0;
-          PF_VF(m) = v;
-          PF_RLAST(m) = rt[m];
-        });
-      }
-      sfor<0, NAQ>([&](auto Q) {
-        constexpr int i = decltype(Q)::value;
-        A.pri_molal[i * ld + c] = x[i];
-        const bool keep = ok && ((small >> i) & 1u);  // original value restored
-        if (!keep) A.total[i * ld + c] = (!ok && restore) ? PF_TINIT(i) : totc[i];
-        if constexpr (NEWTON_ACT) A.pri_act_coef[i * ld + c] = pf_exp(PF_LNGAM(i));
-      });
-      sfor<0, NIMM>([&](auto Q) {
-        constexpr int i = NAQ + decltype(Q)::value;
-        const bool keep = ok && ((small >> i) & 1u);
-        if (!keep) A.immobile[(i - NAQ) * ld + c] = (!ok && restore) ? PF_TINIT(i) : x[i];
-      });
-      sfor<0, NM>([&](auto M) {
-        constexpr int m = decltype(M)::value;
-        A.mnrl_volfrac[m * ld + c] = PF_VF(m);
-        if (A.mnrl_rate) A.mnrl_rate[m * ld + c] = PF_RLAST(m);
-      });
-      if constexpr (NEWTON_ACT && Net::ACT_H2O) {
-        if (A.ln_act_h2o) A.ln_act_h2o[c] = ln_aw;
-      }
-      if (A.num_iterations) A.num_iterations[c] = nit_total;
-      if (A.num_sub_steps) A.num_sub_steps[c] = nsub;
-      if (A.status) A.status[c] = status;
-      cell = -1;
-      mode = 0;
-      continue;
-    }
-
     if constexpr (NEWTON_ACT) {
       sec_I = nsI;
       sec_sum = nss;
@@ -660,39 +922,41 @@ __device__ __forceinline__ void lane_step(const Args& A) {
     }
     if (outcome == 0) {
       // ---------------- linear solve (RSolve) ----------------
-      // aqueous block: A = D^-1/2 M D^-1/2, L D L^T, A y = D^-1/2 res / jc
+      // aqueous block M delta = res / jc by L D L^T.  SCALED: symmetric
+      // scaling to (about) unit diagonal, A = D^-1/2 M D^-1/2; any positive s
+      // gives the same step, so the hardware estimate of 1/sqrt(D_i) is
+      // used.  FP64 needs no scaling (the elimination's relative rounding
+      // does not depend on it); the pivot test is relative to each diagonal.
+      constexpr bool SCALED = F32 || !Net::ANY_PROD;
+      JT a[NT], dg[NA1], b[NA1], dinv[NA1], piv0[NA1], rr[NA1];
       double s[NA1];
-      JT rr[NA1], b[NA1], dg0[NA1];
       const double ijs = wet ? ijc : 1.0;
+      bool bad = false;
       sfor<0, NAQ>([&](auto Q) {
         constexpr int i = decltype(Q)::value;
-        // symmetric scaling to (about) unit diagonal: any positive s gives
-        // the same step, so the hardware estimate of 1/sqrt(D_i) is used
-        s[i] = __builtin_amdgcn_rsq(D[i]);
-        rr[i] = F32 ? (JT)(s[i] * rcp_nr(sig[i])) : (JT)s[i];  // ~sqrt(x_i / D_i)
-        dg0[i] = (JT)(D[i] * s[i] * s[i]);
-        b[i] = (JT)(res[i] * s[i] * ijs);
-      });
-      JT a[NT], dinv[NA1];
-#pragma unroll
-      for (int q = 0; q < NT; ++q) a[q] = (JT)0;
-      sfor<1, NAQ>([&](auto Q) {
-        constexpr int i = decltype(Q)::value;
+        if constexpr (SCALED) {
+          s[i] = __builtin_amdgcn_rsq(D[i]);
+          rr[i] = F32 ? (JT)(s[i] * rcp_nr(sig[i])) : (JT)s[i];  // ~sqrt(x_i / D_i)
+          dg[i] = (JT)(D[i] * s[i] * s[i]);
+          b[i] = (JT)(res[i] * s[i] * ijs);
+          piv0[i] = (JT)kPivTol;
+        } else {
+          dg[i] = D[i];
+          b[i] = res[i] * ijs;
+          piv0[i] = D[i] * kPivTol;
+        }
         sfor<0, i>([&](auto Q2) {
           constexpr int j = decltype(Q2)::value;
-          a[tri(i, j)] = S[tri(i, j)] * rr[i] * rr[j];
+          if constexpr (SCALED) a[tri(i, j)] = S[tri(i, j)] * rr[i] * rr[j];
+          else a[tri(i, j)] = S[tri(i, j)];
         });
       });
-      bool bad = false;
-      // right-looking L D L^T on the unit-diagonal matrix
-      JT dg[NA1];
-#pragma unroll
-      for (int i = 0; i < NA1; ++i) dg[i] = dg0[i];
+      // right-looking
       sfor<0, NAQ>([&](auto P) {
         constexpr int p = decltype(P)::value;
         const JT dp = dg[p];
-        if (!((double)dp > kPivTol)) bad = true;
-        const JT inv = (JT)1 / dp;
+        if (!((double)dp > (double)piv0[p])) bad = true;  // also for a NaN
+        const JT inv = SCALED ? (JT)1 / dp : (JT)rcp_nr((double)dp);
         dinv[p] = inv;
         JT l[NA1];
         sfor<p + 1, NAQ>([&](auto Q) {
@@ -734,7 +998,7 @@ __device__ __forceinline__ void lane_step(const Args& A) {
       double delta[N];
       sfor<0, NAQ>([&](auto Q) {
         constexpr int i = decltype(Q)::value;
-        delta[i] = (double)b[i] * s[i];
+        delta[i] = SCALED ? (double)b[i] * s[i] : (double)b[i];
         if (!(delta[i] == delta[i])) bad = true;
       });
       // immobile rows: accumulation + decay on the diagonal
@@ -757,12 +1021,20 @@ __device__ __forceinline__ void lane_step(const Args& A) {
         outcome = 3;
       } else {
         // ---------------- update (reaction.F90:3977-4049) ----------------
-        double latest[N];
+        double latest[N], rc = -1.0;
+        // The small-step exit holds for the FP32 factorization too: scaled
+        // to unit diagonal, M has |M_ij| <= 1 (positive semi-definite
+        // terms), so |M| <= n and a step below the tolerance certifies a
+        // scaled FP64 residual |b| <= n |y| of the same size.
         if constexpr (Net::LOG_FORM) {
 #pragma unroll
           for (int i = 0; i < N; ++i) {
             const double u = copysign(1.0, delta[i]) * fmin(fabs(delta[i]), Net::MAX_DLNC);
-            latest[i] = x[i] * pf_exp(-u);
+            const double f = exp_step(-u);
+            latest[i] = x[i] * f;
+            // |latest - x| / x
+            const double q = Net::ANY_PROD ? fabs(f - 1.0) : fabs((latest[i] - x[i]) * rcp_nr(x[i]));
+            if (q == q) rc = fmax(rc, q);
           }
         } else {
           double ratio = 1.0e308;
@@ -770,18 +1042,12 @@ __device__ __forceinline__ void lane_step(const Args& A) {
           for (int i = 0; i < N; ++i)
             if (x[i] <= delta[i]) ratio = fmin(ratio, fabs(x[i] / delta[i]));
 #pragma unroll
-          for (int i = 0; i < N; ++i) latest[i] = x[i] - (ratio < 1.0 ? delta[i] * ratio * 0.99 : delta[i]);
+          for (int i = 0; i < N; ++i) {
+            latest[i] = x[i] - (ratio < 1.0 ? delta[i] * ratio * 0.99 : delta[i]);
+            const double q = fabs((latest[i] - x[i]) * rcp_nr(x[i]));
+            if (q == q) rc = fmax(rc, q);
+          }
         }
-        double rc = -1.0;
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          const double q = fabs((latest[i] - x[i]) * rcp_nr(x[i]));
-          if (q == q) rc = fmax(rc, q);
-        }
-        // The small-step exit holds for the FP32 factorization too: the
-        // scaled matrix has unit diagonal and |A_ij| <= 1 (positive
-        // semi-definite terms), so |A| <= n and a step below the tolerance
-        // certifies a scaled FP64 residual |b| <= n |y| of the same size.
         if (polish) {
 #pragma unroll
           for (int i = 0; i < N; ++i) x[i] = latest[i];
@@ -832,7 +1098,7 @@ __device__ __forceinline__ void lane_step(const Args& A) {
     } else if (outcome == 3 || (outcome == 2 && F32 && A.escalate)) {
       // hand the untouched cell to the next pass
       if (A.escalate) {
-        A.status[c] = kEscalate;
+        hand_over(A, c);
         cell = -1;
         mode = 0;
         continue;
@@ -874,7 +1140,7 @@ __device__ __forceinline__ void lane_step(const Args& A) {
   }
 #undef PF_GUESS
 #undef PF_TINIT
-#undef PF_LNGAM
+#undef PF_GAM
 #undef PF_VF
 #undef PF_AREA
 #undef PF_RLAST
@@ -1053,10 +1319,10 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
       A.status[c] = 4;  // PFCHEM_CELL_SENS_UNSUPPORTED
       return;
     }
-    double lng[NA1], gi[NG1], area[NM1], vf[NM1];
+    double gam[NA1], gi[NG1], area[NM1], vf[NM1];
     sfor<0, NAQ>([&](auto Q) {
       constexpr int i = decltype(Q)::value;
-      lng[i] = pf_log(A.pri_act_coef[i * ld + c]);
+      gam[i] = act_keep(A.pri_act_coef[i * ld + c]);
     });
     bool cons = true;
     {
@@ -1084,33 +1350,22 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
       vf[m] = A.mnrl_volfrac[m * ld + c];
       area[m] = A.mnrl_area[m * ld + c];
     });
-    // secondary molality of complex K at ln activities lna
-    auto cplx_m = [&](auto K, const double(&lna)[NA1]) {
+    // secondary molality of complex K at the activities ac
+    auto cplx_m = [&](auto K, const Acts<NA1>& ac) {
       constexpr int k = decltype(K)::value;
-      double lnQK = cplx_lnk<k>(lnT, tk);
-      if constexpr (Net::CPLX_H2O[k] != 0.0) lnQK += Net::CPLX_H2O[k] * ln_aw;
-      sfor<0, Net::CPLX_N[k]>([&](auto Q) {
-        constexpr int a = decltype(Q)::value;
-        lnQK += Net::CPLX_NU[k][a] * lna[Net::CPLX_ID[k][a]];
-      });
-      double m = pf_exp(lnQK);
-      if constexpr (Net::CPLX_GCLS[k] >= 0) m *= gi[Net::CPLX_GCLS[k]];
-      return m;
+      if constexpr (Net::CPLX_GCLS[k] >= 0)
+        return cplx_q<k>(ac, lnT, tk, ln_aw, gi[Net::CPLX_GCLS[k]]);
+      else
+        return cplx_q<k>(ac, lnT, tk, ln_aw, 1.0);
     };
-    // rate of mineral M at lna with volume fraction v: Im, dIm/dlnQK
-    auto mnrl_r = [&](auto Mq, const double(&lna)[NA1], double v, double& Im, double& dI) {
+    // rate of mineral M at ac with volume fraction v: Im, dIm/dlnQK
+    auto mnrl_r = [&](auto Mq, const Acts<NA1>& ac, double v, double& Im, double& dI) {
       constexpr int mi = decltype(Mq)::value;
-      double lnQK = mnrl_lnk<mi>(lnT, tk);
-      if constexpr (Net::MNRL_H2O[mi] != 0.0) lnQK += Net::MNRL_H2O[mi] * ln_aw;
-      sfor<0, Net::MNRL_N[mi]>([&](auto Q) {
-        constexpr int a = decltype(Q)::value;
-        lnQK += Net::MNRL_NU[mi][a] * lna[Net::MNRL_ID[mi][a]];
-      });
       Im = 0.0;
       dI = 0.0;
       if (area[mi] == 0.0) return false;
-      const double QK = pf_exp(lnQK);
-      const MRate r = mineral_rate<mi>(lnQK, QK, v, area[mi], temp);
+      const double QK = mnrl_q<mi>(ac, lnT, tk, ln_aw);
+      const MRate r = mineral_rate<mi>(QK, v, area[mi], temp);
       if (!r.active) return false;
       Im = r.Im;
       dI = r.dIm * QK;
@@ -1121,11 +1376,12 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
     auto system = [&](const double(&x)[NA1], const double(&T0)[NA1], const double(&v0)[NM1],
                       double h, double mf, double(&T)[NA1], double(&res)[NA1], double(&D)[NA1],
                       double(&S)[NT]) {
-      double lna[NA1], tot[NA1];
+      Acts<NA1> ac;
+      double tot[NA1];
       const double jc = psv * dkl / h;
       sfor<0, NAQ>([&](auto Q) {
         constexpr int i = decltype(Q)::value;
-        lna[i] = pf_log(x[i]) + lng[i];
+        act_set<i>(ac, x[i], gam[i]);
         tot[i] = 0.0;
         D[i] = x[i];
       });
@@ -1134,7 +1390,7 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
       sfor<0, NC>([&](auto K) {
         constexpr int k = decltype(K)::value;
         constexpr int ns = Net::CPLX_N[k];
-        const double m = cplx_m(K, lna);
+        const double m = cplx_m(K, ac);
         sfor<0, ns>([&](auto Q) {
           constexpr int a = decltype(Q)::value;
           constexpr int ia = Net::CPLX_ID[k][a];
@@ -1159,7 +1415,7 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
         constexpr int mi = decltype(Mq)::value;
         constexpr int ns = Net::MNRL_N[mi];
         double Im, dI;
-        if (!mnrl_r(Mq, lna, v0[mi], Im, dI)) return;
+        if (!mnrl_r(Mq, ac, v0[mi], Im, dI)) return;
         const double g = dI * vol * mf / jc;
         sfor<0, ns>([&](auto Q) {
           constexpr int a = decltype(Q)::value;
@@ -1281,16 +1537,16 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
       });
       // kinetic update with the rates at the sub-step's solution
       {
-        double lna[NA1];
+        Acts<NA1> ac;
         sfor<0, NAQ>([&](auto Q) {
           constexpr int i = decltype(Q)::value;
-          lna[i] = pf_log(x[i]) + lng[i];
+          act_set<i>(ac, x[i], gam[i]);
         });
         sfor<0, NM>([&](auto Mq) {
           constexpr int mi = decltype(Mq)::value;
           lg[(NAQ + mi) * ldl] = vf[mi];
           double Im, dI;
-          mnrl_r(Mq, lna, vf[mi], Im, dI);
+          mnrl_r(Mq, ac, vf[mi], Im, dI);
           double v = vf[mi] + Im * Net::MNRL_VM[mi] * tdt;
           vf[mi] = v < 0.0 ? 0.0 : v;
         });
@@ -1321,10 +1577,10 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
     // ---------------- objective and its explicit terms ----------------
     double gm[NA1], gT[NA1], gV[NM1];
     {
-      double lna[NA1];
+      Acts<NA1> ac;
       sfor<0, NAQ>([&](auto Q) {
         constexpr int i = decltype(Q)::value;
-        lna[i] = pf_log(x[i]) + lng[i];
+        act_set<i>(ac, x[i], gam[i]);
         gm[i] = 0.0;
         gT[i] = 0.0;
       });
@@ -1338,7 +1594,7 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
         constexpr int k = decltype(K)::value;
         const double wk = A.ws[k];
         if (wk == 0.0) return;
-        const double mk = cplx_m(K, lna);
+        const double mk = cplx_m(K, ac);
         f += wk * mk;
         sfor<0, Net::CPLX_N[k]>([&](auto Q) {
           constexpr int a = decltype(Q)::value;
@@ -1354,11 +1610,12 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
     for (int k = nlog - 1; k >= 0; --k) {
       const bool first = k == nlog - 1;
       const double* lg = A.log + (i64)k * NF * ldl + c;
-      double m[NA1], v0[NM1], lna[NA1];
+      Acts<NA1> ac;
+      double m[NA1], v0[NM1];
       sfor<0, NAQ>([&](auto Q) {
         constexpr int i = decltype(Q)::value;
         m[i] = lg[i * ldl];
-        lna[i] = pf_log(m[i]) + lng[i];
+        act_set<i>(ac, m[i], gam[i]);
       });
       sfor<0, NM>([&](auto M) {
         constexpr int mi = decltype(M)::value;
@@ -1372,7 +1629,7 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
       sfor<0, NM>([&](auto Mq) {
         constexpr int mi = decltype(Mq)::value;
         double Im, dI;
-        actq[mi] = mnrl_r(Mq, lna, v0[mi], Im, dI);
+        actq[mi] = mnrl_r(Mq, ac, v0[mi], Im, dI);
         Imq[mi] = Im;
         gkin[mi] = 0.0;
         if (v0[mi] + Im * Net::MNRL_VM[mi] * h < 0.0) gV[mi] = 0.0;
@@ -1407,7 +1664,7 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
           dotT += Net::CPLX_NU[kk][a] * gT[Net::CPLX_ID[kk][a]];
         });
         if (dotT == 0.0) return;
-        const double mk = cplx_m(K, lna);
+        const double mk = cplx_m(K, ac);
         sfor<0, ns>([&](auto Q) {
           constexpr int a = decltype(Q)::value;
           gt[Net::CPLX_ID[kk][a]] += Net::CPLX_NU[kk][a] * mk * dotT;
@@ -1443,7 +1700,7 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
           if (first) *o = 0.0;
           return;
         }
-        const double mk = cplx_m(K, lna);
+        const double mk = cplx_m(K, ac);
         const double v = (accT - psv / h * accL) * (-kLogToLn * mk * dkl) + wk * (-kLogToLn * mk);
         *o = first ? v : *o + v;
       });

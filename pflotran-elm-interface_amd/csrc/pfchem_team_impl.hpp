@@ -569,6 +569,9 @@ team_step_kernel(const DevNet* np, const DevState* sp, int64_t ncell, double dt,
   // earlier pass handed over)
   const bool listed = s.cell_list != nullptr;
   const int64_t nwork = listed ? (int64_t)gld(s.list_count) : ncell;
+  // an empty list (a step that handed no cell over): trying every XCD's
+  // range for it took the grid 65 us
+  if (nwork == 0) return;
   const int64_t chunk = (nwork + nxcd - 1) / nxcd;
 
   // team-uniform cell state
@@ -1338,7 +1341,8 @@ __global__ void zero_cursors(unsigned long long* c, int n) {
 template <int L, int R, typename JT, int SD, bool VAR>
 hipError_t launch_LR(const DevNet& n, const DevNet* dn, const DevState* ds, int64_t ncell,
                      double dt, const LaunchCfg& cfg, unsigned long long* cursors,
-                     int num_cus, int nxcd, hipStream_t stream, int rescue_only) {
+                     int num_cus, int nxcd, hipStream_t stream, int rescue_only,
+                     bool cursors_clear = false) {
   const TeamLds lay = team_lds_layout(L * R, n.nc, n.nm, 8, sd_lds_doubles(n.sd.nrxn, SD));
   const int block = cfg.block_size;
   const size_t lds = (size_t)(block / L) * lay.bytes;
@@ -1354,7 +1358,7 @@ hipError_t launch_LR(const DevNet& n, const DevNet* dn, const DevState* ds, int6
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
   }
-  zero_cursors<<<1, 64, 0, stream>>>(cursors, nxcd);
+  if (!cursors_clear) zero_cursors<<<1, 64, 0, stream>>>(cursors, nxcd);
   team_step_kernel<L, R, JT, SD, VAR><<<dim3((unsigned)blocks), dim3(block), lds, stream>>>(
       dn, ds, ncell, dt, cursors, nxcd, rescue_only);
   return hipGetLastError();
@@ -1362,7 +1366,8 @@ hipError_t launch_LR(const DevNet& n, const DevNet* dn, const DevState* ds, int6
 
 // mixed = 0: FP64 variant; 1: mixed variant (FP32 pass, then an FP64 pass
 // over the cells the FP32 pass handed over); kTeamRescue64: only the FP64
-// pass over cells an earlier pass handed over (status kEscalate)
+// pass over cells an earlier pass handed over (status kEscalate), on cursors
+// the caller has cleared
 template <int L, int R, int SD, bool VAR>
 hipError_t launch_variant(const DevNet& n, const DevNet* dn, const DevState* ds, int64_t ncell,
                           double dt, int mixed, const LaunchCfg& cfg,
@@ -1372,7 +1377,7 @@ hipError_t launch_variant(const DevNet& n, const DevNet* dn, const DevState* ds,
     LaunchCfg c64 = cfg;
     while (c64.block_size > 64 && !team_supports(n, c64, false)) c64.block_size /= 2;
     return launch_LR<L, R, double, SD, VAR>(n, dn, ds, ncell, dt, c64, cursors, num_cus, nxcd,
-                                            stream, 1);
+                                            stream, 1, true);
   }
   if (!mixed)
     return launch_LR<L, R, double, SD, VAR>(n, dn, ds, ncell, dt, cfg, cursors, num_cus, nxcd,
