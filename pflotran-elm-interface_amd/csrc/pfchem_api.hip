@@ -75,6 +75,10 @@ struct pfchem_ctx {
   std::string lane_src;
   bool lane_ok = false;
   bool lane_ready = false;
+  // a SomDec network the step kernel takes: it runs until a launch shape is
+  // set (launch holds the team shape of the pass over handed-over cells)
+  bool sd_lane = false;
+  bool launch_set[3] = {};
   std::string lane_why;
   std::string lane_adj_src;  // the adjoint module's source (compiled at first use)
   bool lane_adj_ready = false;
@@ -756,6 +760,9 @@ int pfchem_create(const pfchem_network* net, const pfchem_options* opt, int devi
     ctx->lane_src = lane_source(net, opt);
     for (int v = PFCHEM_KERNEL_BATCHED_FP64; v <= PFCHEM_KERNEL_BATCHED_MIXED; ++v)
       ctx->launch[v] = LaunchCfg{1, 1, 256, 0, ctx->max_lds};
+  } else if (lane_sd_supported(net, opt)) {
+    ctx->sd_lane = true;
+    ctx->lane_src = lane_source(net, opt);
   }
   if (hipMalloc(&ctx->dnet_dev, sizeof(DevNet)) != hipSuccess ||
       hipMalloc(&ctx->dstate_ring, sizeof(DevState) * kStateRing) != hipSuccess ||
@@ -790,7 +797,7 @@ TuneInfo tune_info(const pfchem_ctx* ctx) {
   t.nkinmnrl = ctx->net.nkinmnrl;
   t.ncomp = d.ncomp;
   t.variable = d.variable;
-  t.lane_ok = ctx->lane_ok;
+  t.lane_ok = ctx->lane_ok || ctx->sd_lane;
   int p2 = 1;
   while (p2 < d.ncomp) p2 *= 2;
   char buf[256];
@@ -897,8 +904,21 @@ static int to_dev_state(pfchem_ctx* ctx, const pfchem_state* st, int64_t ncell, 
 // latency of its slowest cell: a team of lanes runs one Newton iteration
 // several times faster than one lane does.
 static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double dt, bool mixed,
+                     hipStream_t s);
+// a captured stream takes no module load and no allocation: a call whose
+// one-lane module or scratch is not there yet keeps the team kernel then
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+static bool sd_lane_now(const pfchem_ctx* ctx, int64_t ncell, const DevState& d, hipStream_t s) {
+  const bool ready = ctx->lane_ready && ncell <= ctx->esc_cap &&
+                     (d.status || ncell <= ctx->status_cap);
+  return ctx->sd_lane && (ready || !capturing(s));
+}
+static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double dt, bool mixed,
                      hipStream_t s) {
-  if (!ctx->lane_ok)
+  if (!ctx->lane_ok && !ctx->sd_lane)
     return fail(ctx, PFCHEM_ERR_UNSUPPORTED, "one-lane kernel: " + ctx->lane_why);
   if (!ctx->lane_ready) {
     std::string msg;
@@ -940,11 +960,15 @@ static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double d
   a.num_iterations = d.num_iterations;
   a.num_sub_steps = d.num_sub_steps;
   a.status = st;
+  a.sd_ft = d.somdec_f_t;
+  a.sd_fw = d.somdec_f_w;
   a.dt = dt;
   a.nxcd = ctx->nxcd;
   a.escalate = 1;
-  const int bpc = ctx->launch[mixed ? PFCHEM_KERNEL_BATCHED_MIXED : PFCHEM_KERNEL_BATCHED_FP64]
-                      .blocks_per_cu;
+  // workgroups per CU: the caps of one-lane shapes
+  const LaunchCfg& l64 = ctx->launch[PFCHEM_KERNEL_BATCHED_FP64];
+  const LaunchCfg& lv = mixed ? ctx->launch[PFCHEM_KERNEL_BATCHED_MIXED] : l64;
+  const int bpc = lv.lanes_per_cell == 1 ? lv.blocks_per_cu : 0;
   hipError_t e = hipSuccess;
   a.rescue = 0;
   // the rescue pass walks only the cells the one-lane pass handed over,
@@ -984,7 +1008,7 @@ static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double d
   }
   if (e != hipSuccess)
     return hip_fail(ctx, e, mixed ? "lane kernel launch (FP32)" : "lane kernel launch (FP64)");
-  if (listed && mixed) {
+  if (listed && mixed && !ctx->sd_lane) {
     // the FP64 one-lane kernel takes the handed-over cells first (it returns
     // at once for an empty list), the team pass what that kernel hands over:
     // a Newton iteration of the team kernel, which reads the network's
@@ -995,13 +1019,13 @@ static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double d
     b.list = a.esc_list;
     b.list_count = ctx->esc_list;
     b.esc_list = nullptr;
-    b.list_min = ctx->net.naqcomp < kProdMinAq ? kLaneListMin : 0;
+    b.list_min = ctx->lane_ok && ctx->net.naqcomp < kProdMinAq ? kLaneListMin : 0;
     e = lane_launch(ctx->lane_src, ctx->device, 0, b, ctx->num_cus,
-                    ctx->launch[PFCHEM_KERNEL_BATCHED_FP64].blocks_per_cu, cursors + 16 * ctx->nxcd,
-                    0, s);
+                    l64.lanes_per_cell == 1 ? l64.blocks_per_cu : 0, cursors + 16 * ctx->nxcd, 0, s);
     if (e != hipSuccess) return hip_fail(ctx, e, "lane kernel launch (FP64 list)");
   }
-  e = launch_team_step(ctx->dnet, ctx->dnet_dev, slot, ncell, dt, kTeamRescue64,
+  e = launch_team_step(ctx->dnet, ctx->dnet_dev, slot, ncell, dt,
+                       mixed && ctx->sd_lane ? kTeamRescueMixed : kTeamRescue64,
                        ctx->team_default, cursors + 32 * ctx->nxcd, ctx->num_cus, ctx->nxcd, s,
                        true);
   if (e == hipSuccess) e = release_slot(ctx, k, s);
@@ -1101,7 +1125,8 @@ int pfchem_step(pfchem_ctx* ctx, int64_t ncell, const pfchem_state* state, doubl
       return PFCHEM_OK;
     }
     const LaunchCfg& cfg = ctx->launch[variant];
-    if (cfg.lanes_per_cell == 1) return lane_step(ctx, ncell, d, dt, mixed, s);
+    if (cfg.lanes_per_cell == 1 || (!ctx->launch_set[variant] && sd_lane_now(ctx, ncell, d, s)))
+      return lane_step(ctx, ncell, d, dt, mixed, s);
     if (!team_supports(ctx->dnet, cfg, mixed))
       return fail(ctx, PFCHEM_ERR_UNSUPPORTED, "launch configuration does not fit this network");
     int k = 0;
@@ -1179,17 +1204,19 @@ int pfchem_set_launch(pfchem_ctx* ctx, int variant, const pfchem_launch* cfg) {
   if (variant != PFCHEM_KERNEL_PLAIN_FP64 && c.lanes_per_cell == 1) {
     // the network-specialized lane kernel: 256-lane workgroups, at most as
     // many per CU as its occupancy allows
-    if (!ctx->lane_ok)
+    if (!ctx->lane_ok && !ctx->sd_lane)
       return fail(ctx, PFCHEM_ERR_UNSUPPORTED, "one-lane kernel: " + ctx->lane_why);
     if (c.rows_per_lane != 1 || c.block_size != 256)
       return fail(ctx, PFCHEM_ERR_INVALID, "the one-lane kernel runs 256-lane workgroups, 1 row");
     ctx->launch[variant] = c;
+    ctx->launch_set[variant] = true;
     return PFCHEM_OK;
   }
   if (variant != PFCHEM_KERNEL_PLAIN_FP64 &&
       !team_supports(ctx->dnet, c, variant == PFCHEM_KERNEL_BATCHED_MIXED))
     return fail(ctx, PFCHEM_ERR_UNSUPPORTED, "launch configuration does not fit this network");
   ctx->launch[variant] = c;
+  ctx->launch_set[variant] = true;
   if (ctx->dnet.variable && variant != PFCHEM_KERNEL_PLAIN_FP64 && c.rows_per_lane == 1)
     for (int b = 0; b < kBuckets; ++b)
       if (kBucketBound[b] == c.lanes_per_cell) ctx->vlaunch[variant - 1][b] = c;

@@ -79,7 +79,9 @@ int team_supports(const DevNet& n, const LaunchCfg& cfg, bool mixed);
 // pass could not converge (needs the per-cell status array); kTeamRescue64:
 // only the FP64 pass over cells whose status is kTeamEscalate (cursors
 // cleared by the caller).
+// kTeamRescueMixed: the FP32 and then the FP64 pass over those cells.
 constexpr int kTeamRescue64 = 2;
+constexpr int kTeamRescueMixed = 3;
 constexpr int kTeamEscalate = 16;
 hipError_t launch_team_step(const DevNet& n, const DevNet* dn, const DevState* ds,
                             int64_t ncell, double dt, int mixed, const LaunchCfg& cfg,

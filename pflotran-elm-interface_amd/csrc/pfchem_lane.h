@@ -49,8 +49,10 @@ struct LaneArgs {
   const int* list_count;
   int* esc_list;
   unsigned long long* esc_count;
+  const double* sd_ft;
+  const double* sd_fw;
 };
-static_assert(sizeof(LaneArgs) == 224, "LaneArgs layout");
+static_assert(sizeof(LaneArgs) == 240, "LaneArgs layout");
 
 // adjoint kernel arguments; the same layout as pflane::SensArgs
 struct LaneSensArgs {
@@ -90,6 +92,10 @@ constexpr int kProdMinAq = 9;
 
 // 1 if the lane kernel handles this network and these options (else `why`)
 int lane_supported(const pfchem_network* net, const pfchem_options* opt, std::string& why);
+// 1 if the step kernel takes this network with its SomDec sandbox (no
+// complexes, minerals, Monod oxygen response, O2 tracking or activity update
+// per Newton iteration)
+int lane_sd_supported(const pfchem_network* net, const pfchem_options* opt);
 // full device source: the network as constants followed by the template
 std::string lane_source(const pfchem_network* net, const pfchem_options* opt);
 // compile `src` for gfx950 and load it on `device` (cached per process)

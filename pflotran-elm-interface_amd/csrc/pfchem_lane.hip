@@ -200,11 +200,159 @@ int lane_supported(const pfchem_network* net, const pfchem_options* opt, std::st
   return 1;
 }
 
+int lane_sd_supported(const pfchem_network* net, const pfchem_options* opt) {
+  const pfchem_somdec* sd = net->somdec;
+  const int naq = net->naqcomp, nimm = net->nimmobile;
+  if (!sd || sd->nrxn < 1 || net->neqcplx > 0 || net->nkinmnrl > 0 || opt->variable_ncomp) return 0;
+  if (naq < 1 || naq > kLaneMaxAq || naq + nimm > 32) return 0;
+  if (2 * (naq + nimm) + naq > kLaneMaxLdsFields) return 0;
+  if (opt->act_coef_update_frequency == PFCHEM_ACT_COEF_FREQUENCY_NEWTON_ITER) return 0;
+  if (sd->species_id_co2 < 0 || sd->species_id_nh4 < 0 || sd->species_o2 != 0) return 0;
+  for (int r = 0; r < sd->nrxn; ++r)
+    if (sd->Ox_response_function[r] == 1) return 0;
+  return 1;
+}
+
+// the sandbox's constants and its Jacobian pattern: every entry
+// pfchem_lane.hpp adds, the diagonal, and the fill-in of the elimination in
+// natural order
+static void sd_source(Gen& g, const pfchem_network* net) {
+  const pfchem_somdec* sd = net->somdec;
+  const int naq = net->naqcomp, N = naq + net->nimmobile, nr = sd->nrxn;
+  const int MD = PFCHEM_SOMDEC_MAX_DOWN, MM = PFCHEM_SOMDEC_MAX_MONOD, MI = PFCHEM_SOMDEC_MAX_INHIB;
+  auto iv = [&](const int32_t* p) { return std::vector<int>(p, p + nr); };
+  auto dv = [&](const double* p) { return std::vector<double>(p, p + nr); };
+  auto im = [&](const int32_t* p, int w) {
+    std::vector<std::vector<int>> m;
+    for (int r = 0; r < nr; ++r) m.emplace_back(p + r * w, p + (r + 1) * w);
+    return m;
+  };
+  auto dm = [&](const double* p, int w) {
+    std::vector<std::vector<double>> m;
+    for (int r = 0; r < nr; ++r) m.emplace_back(p + r * w, p + (r + 1) * w);
+    return m;
+  };
+  g.i("SDN", nr);
+  g.i("SD_CO2", sd->species_id_co2);
+  g.i("SD_NH4", sd->species_id_nh4);
+  g.i("SD_NO3", sd->species_id_no3);
+  g.i("SD_N2O", sd->species_id_n2o);
+  g.i("SD_PROTON", sd->species_id_proton);
+  g.i("SD_HR", sd->species_id_hr);
+  g.i("SD_NMIN", sd->species_id_nmin);
+  g.i("SD_NIMM", sd->species_id_nimm);
+  g.i("SD_NIMP", sd->species_id_nimp);
+  g.i("SD_NGASMIN", sd->species_id_ngasmin);
+  g.d("SD_X0EPS", sd->x0eps);
+  g.d("SD_N2OFRAC", sd->n2o_frac_mineralization);
+  g.d("SD_INHIB", sd->inhibition_nh4_no3);
+  g.dvec("SD_K0", dv(sd->rate_constant));
+  g.dvec("SD_KD", dv(sd->rate_decomposition));
+  g.dvec("SD_AD", dv(sd->rate_ad_factor));
+  g.ivec("SD_UC", iv(sd->upstream_c_id));
+  g.ivec("SD_UN", iv(sd->upstream_n_id));
+  g.ivec("SD_UHR", iv(sd->upstream_hr_id));
+  g.ivec("SD_UNMIN", iv(sd->upstream_nmin_id));
+  g.ivec("SD_UNIMP", iv(sd->upstream_nimp_id));
+  g.ivec("SD_UNIMM", iv(sd->upstream_nimm_id));
+  g.dvec("SD_UNC", dv(sd->upstream_nc));
+  g.ivec("SD_VARY", iv(sd->upstream_is_varycn));
+  g.ivec("SD_ND", iv(sd->n_downstream_pools));
+  g.imat("SD_DC", im(sd->downstream_c_id, MD), MD);
+  g.imat("SD_DN", im(sd->downstream_n_id, MD), MD);
+  g.dmat("SD_DS", dm(sd->downstream_stoich, MD), MD);
+  g.dmat("SD_DNC", dm(sd->downstream_nc, MD), MD);
+  g.imat("SD_DVARY", im(sd->downstream_is_varycn, MD), MD);
+  g.dvec("SD_MCS", dv(sd->mineral_c_stoich));
+  g.dvec("SD_MNS", dv(sd->mineral_n_stoich));
+  g.ivec("SD_NMON", iv(sd->n_monod));
+  g.imat("SD_MSP", im(sd->monod_specid, MM), MM);
+  g.dmat("SD_MHS", dm(sd->monod_half_saturation, MM), MM);
+  g.dmat("SD_MTH", dm(sd->monod_threshold, MM), MM);
+  g.imat("SD_MPN", im(sd->monod_pool_normalized, MM), MM);
+  g.ivec("SD_NINH", iv(sd->n_inhibition));
+  g.imat("SD_ISP", im(sd->inhibition_specid, MI), MI);
+  g.imat("SD_ITY", im(sd->inhibition_type, MI), MI);
+  g.dmat("SD_IC1", dm(sd->inhibition_constant, MI), MI);
+  g.dmat("SD_IC2", dm(sd->inhibition_constant2, MI), MI);
+  // response classes: (temperature function, its parameter); moisture
+  // function (bit 0) and water-filled pore space (bit 1)
+  std::vector<int> ft, fw, tc(nr), wc(nr);
+  std::vector<double> fp;
+  for (int r = 0; r < nr; ++r) {
+    int t = sd->temperature_response_function[r];
+    if (t < 1 || t > 4) t = 0;
+    const double p = t == 4 ? sd->Ea[r] : t >= 2 ? sd->Q10[r] : 0.0;
+    size_t q = 0;
+    while (q < ft.size() && !(ft[q] == t && fp[q] == p)) ++q;
+    if (q == ft.size()) {
+      ft.push_back(t);
+      fp.push_back(p);
+    }
+    tc[r] = (int)q;
+    const int w = (sd->moisture_response_function[r] == 3 ? 1 : 0) +
+                  (sd->Ox_response_function[r] == 2 ? 2 : 0);
+    q = 0;
+    while (q < fw.size() && fw[q] != w) ++q;
+    if (q == fw.size()) fw.push_back(w);
+    wc[r] = (int)q;
+  }
+  g.i("SD_NFT", (long)ft.size());
+  g.i("SD_NFW", (long)fw.size());
+  g.ivec("SD_FT_TYPE", ft);
+  g.dvec("SD_FT_PAR", fp);
+  g.ivec("SD_FW_TYPE", fw);
+  g.ivec("SD_TCLS", tc);
+  g.ivec("SD_WCLS", wc);
+  // Jacobian pattern
+  std::vector<std::vector<int>> pos(N, std::vector<int>(N, -1));
+  auto put = [&](int row, int col) {
+    if (row >= 0 && col >= 0) pos[row][col] = 0;
+  };
+  auto dof = [&](int imm) { return imm >= 0 ? naq + imm : -1; };
+  for (int i = 0; i < N; ++i) put(i, i);
+  const int nh4 = sd->species_id_nh4, no3 = sd->species_id_no3;
+  for (int r = 0; r < nr; ++r) {
+    const bool vary = sd->upstream_is_varycn[r] != 0;
+    const int uc = dof(sd->upstream_c_id[r]);
+    for (int col : {uc, nh4, no3}) {
+      if (col != uc && !(vary || sd->mineral_n_stoich[r] < 0.0)) continue;
+      if (col == uc || sd->species_id_co2 == col) put(sd->species_id_co2, col);
+      put(uc, col);
+      put(dof(sd->upstream_hr_id[r]), col);
+      put(dof(sd->species_id_hr), col);
+      if (col == uc) put(nh4, col), put(no3, col);
+      put(dof(sd->upstream_nmin_id[r]), col);
+      put(dof(sd->species_id_nmin), col);
+      put(dof(sd->upstream_nimm_id[r]), col);
+      put(dof(sd->species_id_nimm), col);
+      if (vary) put(dof(sd->upstream_n_id[r]), col);
+      for (int j = 0; j < sd->n_downstream_pools[r]; ++j) {
+        put(dof(sd->downstream_c_id[r * MD + j]), col);
+        if (sd->downstream_is_varycn[r * MD + j]) put(dof(sd->downstream_n_id[r * MD + j]), col);
+      }
+    }
+  }
+  if (sd->species_id_n2o >= 0) put(dof(sd->species_id_ngasmin), nh4);
+  for (int p = 0; p < N; ++p)
+    for (int i = p + 1; i < N; ++i)
+      if (pos[i][p] >= 0)
+        for (int j = p + 1; j < N; ++j)
+          if (pos[p][j] >= 0) pos[i][j] = 0;
+  int nnz = 0;
+  for (auto& row : pos)
+    for (int& q : row)
+      if (q >= 0) q = nnz++;
+  g.i("JNNZ", nnz);
+  g.imat("JPOS", pos, N);
+}
+
 std::string lane_source(const pfchem_network* net, const pfchem_options* opt) {
   const int naq = net->naqcomp, nimm = net->nimmobile, nc = net->neqcplx, nm = net->nkinmnrl;
   Gen g;
   // (hiprtc provides the HIP device runtime without an include)
   g.line("// generated: one reaction network and its solver options as constants");
+  if (net->somdec) g.line("#define PFLANE_SD 1");
   g.line("struct Net {");
   g.i("NAQ", naq);
   g.i("NIMM", nimm);
@@ -347,6 +495,8 @@ std::string lane_source(const pfchem_network* net, const pfchem_options* opt) {
     did.push_back(net->decayspecid[r]);
     dk.push_back(net->decay_rate_constant[r]);
   }
+  g.i("HAS_SD", net->somdec ? 1 : 0);
+  if (net->somdec) sd_source(g, net);
   g.ivec("DECAY_ID", did);
   g.dvec("DECAY_K", dk);
   g.line("};");
@@ -364,15 +514,18 @@ int lane_compile(const std::string& src, int device, std::string& err) {
   Module m;
   hipError_t e = hipSetDevice(device);
   if (e == hipSuccess) e = hipModuleLoadData(&m.mod, code.data());
-  // a step module holds the two step kernels, an adjoint module the adjoint
-  const bool adjoint = src.compare(0, sizeof(kLaneAdjointDefine) - 1, kLaneAdjointDefine) == 0;
-  if (e == hipSuccess && adjoint) e = hipModuleGetFunction(&m.adj, m.mod, "pfchem_lane_adjoint");
-  if (e == hipSuccess && !adjoint) e = hipModuleGetFunction(&m.f32, m.mod, "pfchem_lane_step_f32");
-  if (e == hipSuccess && !adjoint) e = hipModuleGetFunction(&m.f64, m.mod, "pfchem_lane_step_f64");
-  if (e == hipSuccess && !adjoint)
-    e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&m.blocks_per_cu32, m.f32, 256, 0);
-  if (e == hipSuccess && !adjoint)
-    e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&m.blocks_per_cu64, m.f64, 256, 0);
+  // a step module holds the two step kernels, the others one kernel each
+  auto kind = [&](const char* define) { return src.compare(0, std::strlen(define), define) == 0; };
+  if (e == hipSuccess && kind(kLaneAdjointDefine)) {
+    e = hipModuleGetFunction(&m.adj, m.mod, "pfchem_lane_adjoint");
+  } else if (e == hipSuccess) {
+    e = hipModuleGetFunction(&m.f32, m.mod, "pfchem_lane_step_f32");
+    if (e == hipSuccess) e = hipModuleGetFunction(&m.f64, m.mod, "pfchem_lane_step_f64");
+    if (e == hipSuccess)
+      e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&m.blocks_per_cu32, m.f32, 256, 0);
+    if (e == hipSuccess)
+      e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&m.blocks_per_cu64, m.f64, 256, 0);
+  }
   if (e != hipSuccess) {
     err = std::string("lane kernel load: ") + hipGetErrorString(e);
     return PFCHEM_ERR_HIP;

@@ -604,6 +604,13 @@ team_step_kernel(const DevNet* np, const DevState* sp, int64_t ncell, double dt,
     // rather than a few waves running the whole list several cells deep
     const int64_t waves = (int64_t)gridDim.x * (blockDim.x / 64);
     if (nwork < 4 * (int64_t)batch * waves) batch = 64 / L;
+    // fewer cells than wavefronts: one cell per wavefront, whose iteration is
+    // shorter without other teams' branches (the pass takes as long as its
+    // slowest cell)
+    if (nwork <= waves) {
+      batch = 1;
+      if (team_in_wave != 0) exhausted = true;
+    }
   }
 
   for (;;) {
@@ -1367,17 +1374,23 @@ hipError_t launch_LR(const DevNet& n, const DevNet* dn, const DevState* ds, int6
 // mixed = 0: FP64 variant; 1: mixed variant (FP32 pass, then an FP64 pass
 // over the cells the FP32 pass handed over); kTeamRescue64: only the FP64
 // pass over cells an earlier pass handed over (status kEscalate), on cursors
-// the caller has cleared
+// the caller has cleared; kTeamRescueMixed: the mixed variant's two passes
+// over those cells
 template <int L, int R, int SD, bool VAR>
 hipError_t launch_variant(const DevNet& n, const DevNet* dn, const DevState* ds, int64_t ncell,
                           double dt, int mixed, const LaunchCfg& cfg,
                           unsigned long long* cursors, int num_cus, int nxcd,
                           hipStream_t stream, bool has_status) {
-  if (mixed == kTeamRescue64) {
+  if (mixed == kTeamRescueMixed) {
+    const hipError_t e = launch_LR<L, R, float, SD, VAR>(n, dn, ds, ncell, dt, cfg, cursors,
+                                                         num_cus, nxcd, stream, 1, true);
+    if (e != hipSuccess) return e;
+  }
+  if (mixed == kTeamRescue64 || mixed == kTeamRescueMixed) {
     LaunchCfg c64 = cfg;
     while (c64.block_size > 64 && !team_supports(n, c64, false)) c64.block_size /= 2;
     return launch_LR<L, R, double, SD, VAR>(n, dn, ds, ncell, dt, c64, cursors, num_cus, nxcd,
-                                            stream, 1, true);
+                                            stream, 1, mixed == kTeamRescue64);
   }
   if (!mixed)
     return launch_LR<L, R, double, SD, VAR>(n, dn, ds, ncell, dt, cfg, cursors, num_cus, nxcd,

@@ -1,0 +1,50 @@
+"""The one-lane SomDec step (the default of networks without complexes,
+minerals and an oxygen response) at cell counts around its wavefront and
+workgroup edges, against the FP64 oracle through the bars of
+test_gpu_somdec.py, and its hand-over to the team kernel."""
+import numpy as np
+import pytest
+
+from pfchem import abi, workloads
+
+import gpu_util as G
+from test_gpu_somdec import FIELDS, VARIANTS, _check, _oracle_band
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ncell,ld", [(1, 1), (63, 64), (65, 65), (257, 300), (4099, 4099)])
+def test_somdec_lane_edges(ncell, ld):
+    wl = workloads.somdec_workload(ncell, ld=ld)
+    ref, rec, nfail = G.run_oracle(wl)
+    assert nfail == 0
+    band = _oracle_band(wl, ref)
+    for variant in VARIANTS:
+        got, _ = G.run_gpu(wl, variant)
+        _check(wl, ref, rec, band, got, "somdec-lane/%d/%s" % (ncell, abi.KERNEL_NAMES[variant]))
+        for f in FIELDS:  # rows beyond the cells stay as they were
+            assert np.array_equal(got[f][:, ncell:], wl.state[f][:, ncell:])
+
+
+@pytest.mark.parametrize("variant", VARIANTS)
+def test_somdec_lane_and_team_agree(variant):
+    """Same cells through the two kernels.  Both end at |step| or residual
+    below the options' tolerances, so they differ where rounding moves that
+    end by an iteration; the oracle's band bounds it, and nearly every cell
+    takes the same sub-steps."""
+    wl = workloads.somdec_workload(20001)
+    lane, ctx = G.run_gpu(wl, variant)
+    assert ctx.get_launch(variant)["lanes_per_cell"] == 16  # the hand-over pass's shape
+    team, _ = G.run_gpu(wl, variant, lanes=16, block=128)
+    one, _ = G.run_gpu(wl, variant, lanes=1, block=256)
+    assert np.all(lane["status"] == 0) and np.all(team["status"] == 0)
+    same = lane["num_sub_steps"] == team["num_sub_steps"]
+    assert (~same).sum() <= 20
+    assert (lane["num_iterations"] != team["num_iterations"]).mean() < 0.01
+    for f in FIELDS:
+        assert np.array_equal(lane[f], one[f]), f  # asked for by shape: the same kernel
+        scale = np.abs(team[f]).max(axis=1, keepdims=True)
+        err = (np.abs(lane[f] - team[f]) / scale)[:, same[0]]
+        # the iteration ends at 1e-8 relative change: one iteration more or
+        # less moves an entry by at most that much of its row's range
+        assert err.max() <= 1e-8, f
