@@ -86,6 +86,34 @@ constexpr int kLaneSensSub = 8;  // sub-steps the adjoint kernel records per cel
 // first line of an adjoint module's source (followed by lane_source)
 constexpr char kLaneAdjointDefine[] = "#define PFLANE_ADJOINT 1\n";
 
+// GIRT block kernel arguments; the same layout as pflane::GirtArgs
+struct LaneGirtArgs {
+  long long ld, ncell;
+  const double* pri_molal;
+  double* total;
+  const double* immobile;
+  double* sec_molal;
+  const double* pri_act_coef;
+  const double* sec_act_coef;
+  const double* ln_act_h2o;
+  const double* mnrl_volfrac;
+  const double* mnrl_area;
+  double* mnrl_rate;
+  const double* porosity;
+  const double* saturation;
+  const double* den_kg;
+  const double* volume;
+  const double* temperature;
+  const double* fixed_total;
+  const double* fixed_imm;
+  double* res;
+  double* jac;
+  double dt;
+};
+static_assert(sizeof(LaneGirtArgs) == 176, "LaneGirtArgs layout");
+// prefix of lane_source that makes a GIRT module
+constexpr char kLaneGirtDefine[] = "#define PFLANE_GIRT 1\n";
+
 // networks of at least this many primaries evaluate mass action as products
 // of powers (pfchem_lane.hpp)
 constexpr int kProdMinAq = 9;
@@ -110,6 +138,9 @@ int lane_compile_only(const std::string& src, std::vector<char>* code, std::stri
 hipError_t lane_launch(const std::string& src, int device, int f32, const LaneArgs& args,
                        int num_cus, int blocks_per_cu, unsigned long long* cursors, int nclear,
                        hipStream_t stream);
+// launch the GIRT kernel of a compiled source, one cell per lane
+hipError_t lane_girt_launch(const std::string& src, int device, const LaneGirtArgs& args,
+                            hipStream_t stream);
 // launch the adjoint kernel of a compiled source, one cell per lane
 hipError_t lane_adjoint_launch(const std::string& src, int device, const LaneSensArgs& args,
                                hipStream_t stream);

@@ -137,7 +137,7 @@ ProdRows prod_rows(const std::vector<std::vector<double>>& nu, const double* log
 
 struct Module {
   hipModule_t mod = nullptr;
-  hipFunction_t f32 = nullptr, f64 = nullptr, adj = nullptr;
+  hipFunction_t f32 = nullptr, f64 = nullptr, adj = nullptr, girt = nullptr;
   int blocks_per_cu32 = 1, blocks_per_cu64 = 1;
 };
 std::mutex g_mu;
@@ -518,6 +518,8 @@ int lane_compile(const std::string& src, int device, std::string& err) {
   auto kind = [&](const char* define) { return src.compare(0, std::strlen(define), define) == 0; };
   if (e == hipSuccess && kind(kLaneAdjointDefine)) {
     e = hipModuleGetFunction(&m.adj, m.mod, "pfchem_lane_adjoint");
+  } else if (e == hipSuccess && kind(kLaneGirtDefine)) {
+    e = hipModuleGetFunction(&m.girt, m.mod, "pfchem_lane_girt");
   } else if (e == hipSuccess) {
     e = hipModuleGetFunction(&m.f32, m.mod, "pfchem_lane_step_f32");
     if (e == hipSuccess) e = hipModuleGetFunction(&m.f64, m.mod, "pfchem_lane_step_f64");
@@ -593,6 +595,24 @@ hipError_t lane_launch(const std::string& src, int device, int f32, const LaneAr
   void* params[] = {&a};
   return hipModuleLaunchKernel(f32 ? m.f32 : m.f64, (unsigned)blocks, 1, 1, 256, 1, 1, 0, stream,
                                params, nullptr);
+}
+
+hipError_t lane_girt_launch(const std::string& src, int device, const LaneGirtArgs& args,
+                            hipStream_t stream) {
+  Module m;
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    auto it = g_mods.find(std::make_pair(device, src));
+    if (it == g_mods.end()) return hipErrorInvalidHandle;
+    m = it->second;
+  }
+  const int64_t blocks = (args.ncell + 63) / 64;
+  if (blocks < 1) return hipSuccess;
+  if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+  LaneGirtArgs a = args;
+  void* params[] = {&a};
+  return hipModuleLaunchKernel(m.girt, (unsigned)blocks, 1, 1, 64, 1, 1, 0, stream, params,
+                               nullptr);
 }
 
 hipError_t lane_adjoint_launch(const std::string& src, int device, const LaneSensArgs& args,

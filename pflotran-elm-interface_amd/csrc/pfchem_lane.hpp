@@ -159,8 +159,16 @@ __device__ __forceinline__ double exp_bounded(double v) {
   p = fma(p, r, 1.0);
   return __builtin_ldexp(p, (int)n);
 }
+// Mass action as products (see Acts below).  The residual and Jacobian block
+// keeps the log form: it is evaluated once a cell, and its totals come from
+// sums that cancel, where the form the caller had before counts.
+#if PFLANE_GIRT
+constexpr bool kProd = false;
+#else
+constexpr bool kProd = Net::ANY_PROD;
+#endif
 __device__ __forceinline__ double exp_step(double v) {
-  if constexpr ((Net::ANY_PROD || Net::HAS_SD) && Net::MAX_DLNC <= 600.0) return exp_bounded(v);
+  if constexpr ((kProd || Net::HAS_SD) && Net::MAX_DLNC <= 600.0) return exp_bounded(v);
   else return pf_exp(v);
 }
 // 1/g by the hardware reciprocal estimate refined with two Newton-Raphson
@@ -226,14 +234,14 @@ struct Acts {
 };
 // ln gamma (networks without product rows) or gamma, as the kernels keep it
 __device__ __forceinline__ double act_keep(double gamma) {
-  if constexpr (Net::ANY_PROD) return gamma;
+  if constexpr (kProd) return gamma;
   else return pf_log(gamma);
 }
 // activity of primary I at molality x; a <= 0 (or NaN) gives NaN, as its
 // logarithm would
 template <int I, int NA1>
 __device__ __forceinline__ void act_set(Acts<NA1>& A, double x, double kept) {
-  if constexpr (!Net::ANY_PROD) {
+  if constexpr (!kProd) {
     A.l[I] = pf_log(x) + kept;
     return;
   }
@@ -258,7 +266,7 @@ __device__ __forceinline__ double ipow(double b) {
 template <int K, int NA1>
 __device__ __forceinline__ double cplx_pe(const Acts<NA1>& A, double lnT, double tk, double ln_aw,
                                           double scale, int& e) {
-  if constexpr (Net::CPLX_PROD[K] != 0) {
+  if constexpr (kProd && Net::CPLX_PROD[K] != 0) {
     double p = Net::CPLX_KM[K] * scale;
     e = Net::CPLX_KE[K];
     sfor<0, Net::CPLX_N[K]>([&](auto Q) {
@@ -285,14 +293,14 @@ __device__ __forceinline__ double cplx_q(const Acts<NA1>& A, double lnT, double 
                                          double scale) {
   int e;
   const double p = cplx_pe<K>(A, lnT, tk, ln_aw, scale, e);
-  if constexpr (Net::CPLX_PROD[K] != 0) return __builtin_ldexp(p, e);
+  if constexpr (kProd && Net::CPLX_PROD[K] != 0) return __builtin_ldexp(p, e);
   else return p;
 }
 // Q/K of kinetic mineral M
 template <int M, int NA1>
 __device__ __forceinline__ double mnrl_q(const Acts<NA1>& A, double lnT, double tk,
                                          double ln_aw) {
-  if constexpr (Net::MNRL_PROD[M] != 0) {
+  if constexpr (kProd && Net::MNRL_PROD[M] != 0) {
     double p = Net::MNRL_KM[M];
     int e = Net::MNRL_KE[M];
     sfor<0, Net::MNRL_N[M]>([&](auto Q) {
@@ -926,7 +934,7 @@ __device__ __forceinline__ void lane_step(const Args& A) {
         *pp = x[i];
         const bool keep = ok && ((small >> i) & 1u);  // original value restored
         if (!keep) *pt = (!ok && restore) ? PF_TINIT(i) : (x[i] + tot[i]) * dkl;
-        if constexpr (NEWTON_ACT) *pa = Net::ANY_PROD ? PF_GAM(i) : pf_exp(PF_GAM(i));
+        if constexpr (NEWTON_ACT) *pa = kProd ? PF_GAM(i) : pf_exp(PF_GAM(i));
         pp += lo;
         pt += lo;
         pa += lo;
@@ -1458,7 +1466,7 @@ __device__ __forceinline__ void lane_step(const Args& A) {
       // gives the same step, so the hardware estimate of 1/sqrt(D_i) is
       // used.  FP64 needs no scaling (the elimination's relative rounding
       // does not depend on it); the pivot test is relative to each diagonal.
-      constexpr bool SCALED = F32 || !Net::ANY_PROD;
+      constexpr bool SCALED = F32 || !kProd;
       JT a[NT], dg[NA1], b[NA1], dinv[NA1], piv0[NA1], rr[NA1];
       double s[NA1];
       const double ijs = wet ? ijc : 1.0;
@@ -1565,7 +1573,7 @@ __device__ __forceinline__ void lane_step(const Args& A) {
             const double f = exp_step(-u);
             latest[i] = x[i] * f;
             // |latest - x| / x
-            const double q = Net::ANY_PROD || SD ? fabs(f - 1.0) : fabs((latest[i] - x[i]) * rcp_nr(x[i]));
+            const double q = kProd || SD ? fabs(f - 1.0) : fabs((latest[i] - x[i]) * rcp_nr(x[i]));
             if (q == q) rc = fmax(rc, q);
           }
         } else {
@@ -1686,10 +1694,9 @@ __device__ __forceinline__ void lane_step(const Args& A) {
 
 }  // namespace pflane
 
-// one module holds either the step kernels or (PFLANE_ADJOINT defined) the
-// adjoint kernel, so a context that never asks for sensitivities does not
-// compile it
-#ifndef PFLANE_ADJOINT
+// one module holds the step kernels, or (PFLANE_ADJOINT defined) the adjoint
+// kernel, or (PFLANE_GIRT) the GIRT block, so a context compiles what it uses
+#if !defined(PFLANE_ADJOINT) && !defined(PFLANE_GIRT)
 extern "C" __global__ void __launch_bounds__(256) pfchem_lane_step_f32(pflane::Args a) {
   pflane::lane_step<float>(a);
 }
@@ -2271,5 +2278,219 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
 #ifdef PFLANE_ADJOINT
 extern "C" __global__ void __launch_bounds__(256) pfchem_lane_adjoint(pflane::SensArgs a) {
   pflane::lane_adjoint(a);
+}
+#endif
+
+// ---------------------------------------------------------------------------
+// GIRT reaction block, one cell per lane, FP64: residual and Jacobian of one
+// iterate (RTResidualNonFlux / RTJacobianNonFlux per cell,
+// reactive_transport.F90:2393-2430, 2599-2642, 3172-3183, 3270-3300), aqueous
+// networks with kinetic minerals and decay.
+//   res_i  = (Acc_i(x) - Acc_i(fixed)) / dt + R_i(x)
+//   jac_ij = (f S_ij + G_ij) / x_j + delta_ij f,  f = dkl psv / dt,
+// S = sum_k nu nu^T m_k and G the minerals' term symmetric: the strict lower
+// triangle and the diagonal stay in registers, then every row of the state
+// leaves as one contiguous 512-byte store of the wavefront.  The kernel is a
+// stream (15 primaries: 3.2 kB a cell): 262,139 cells move 0.84 GB in
+// 286 us; the team kernel, whose LDS atomics and dense-tile write-out cost
+// more than its traffic, took 1190 us.
+namespace pflane {
+
+struct GirtArgs {
+  i64 ld, ncell;
+  const double* pri_molal;
+  double* total;
+  const double* immobile;
+  double* sec_molal;
+  const double* pri_act_coef;
+  const double* sec_act_coef;
+  const double* ln_act_h2o;
+  const double* mnrl_volfrac;
+  const double* mnrl_area;
+  double* mnrl_rate;
+  const double* porosity;
+  const double* saturation;
+  const double* den_kg;
+  const double* volume;
+  const double* temperature;
+  const double* fixed_total;
+  const double* fixed_imm;
+  double* res;
+  double* jac;  // NULL: residual only
+  double dt;
+};
+static_assert(sizeof(GirtArgs) == 176, "GirtArgs layout");
+
+__device__ inline void lane_girt(const GirtArgs& A) {
+  constexpr int NAQ = Net::NAQ, NIMM = Net::NIMM, N = NAQ + NIMM, NC = Net::NC, NM = Net::NM;
+  constexpr int NA1 = NAQ > 0 ? NAQ : 1, NI1 = NIMM > 0 ? NIMM : 1, NM1 = NM > 0 ? NM : 1;
+  constexpr int NC1 = NC > 0 ? NC : 1, NT = NAQ > 1 ? NAQ * (NAQ - 1) / 2 : 1;
+  const i64 c = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= A.ncell) return;
+  const i64 ld = A.ld;
+  // every load first
+  const double por = A.porosity[c], sat = A.saturation[c], den = A.den_kg[c], vol = A.volume[c];
+  const double temp = A.temperature ? A.temperature[c] : 25.0;
+  const double ln_aw = (Net::ACT_H2O && A.ln_act_h2o) ? A.ln_act_h2o[c] : 0.0;
+  double x[N], gam[NA1], fx[N], vf[NM1], ar[NM1], g[NC1];
+  {
+    const double* pp = A.pri_molal + c;
+    const double* pg = A.pri_act_coef + c;
+    const double* pf = A.fixed_total + c;
+    sfor<0, NAQ>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      x[i] = *pp;
+      gam[i] = *pg;
+      fx[i] = *pf;
+      pp += ld;
+      pg += ld;
+      pf += ld;
+    });
+    sfor<0, NIMM>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      x[NAQ + i] = A.immobile[i * ld + c];
+      fx[NAQ + i] = A.fixed_imm[i * ld + c];
+    });
+    const double* pv = A.mnrl_volfrac + c;
+    const double* pa = A.mnrl_area + c;
+    sfor<0, NM>([&](auto M) {
+      constexpr int m = decltype(M)::value;
+      vf[m] = *pv;
+      ar[m] = *pa;
+      pv += ld;
+      pa += ld;
+    });
+    const double* ps = A.sec_act_coef + c;
+    sfor<0, NC>([&](auto K) {
+      g[decltype(K)::value] = *ps;
+      ps += ld;
+    });
+  }
+  issue_loads();
+  const bool wet = !(sat < kRtMinSat);
+  const double dkl = den * 1.0e-3, psv = por * sat * 1000.0 * vol;
+  const double tk = temp + 273.15, lnT = pf_log(tk);
+  const double f = wet ? dkl * (psv / A.dt) : 0.0;
+  Acts<NA1> act;
+  double tot[NA1], D[NA1], W[NT], xi[NA1], res[N];
+  sfor<0, NAQ>([&](auto I) {
+    constexpr int i = decltype(I)::value;
+    act_set<i>(act, x[i], act_keep(gam[i]));
+    xi[i] = 1.0 / x[i];
+    tot[i] = 0.0;
+    D[i] = 0.0;
+  });
+#pragma unroll
+  for (int q = 0; q < NT; ++q) W[q] = 0.0;
+  {
+    double* ps = A.sec_molal + c;
+    sfor<0, NC>([&](auto K) {
+      constexpr int k = decltype(K)::value;
+      constexpr int ns = Net::CPLX_N[k];
+      const double m = cplx_q<k>(act, lnT, tk, ln_aw, 1.0) * rcp_nr(g[k]);
+      *ps = m;
+      ps += ld;
+      const double mf = m * f;
+      sfor<0, ns>([&](auto Q) {
+        constexpr int a = decltype(Q)::value;
+        constexpr int ia = Net::CPLX_ID[k][a];
+        constexpr double na = Net::CPLX_NU[k][a];
+        tot[ia] += na * m;
+        D[ia] += (na * na) * mf;
+        sfor<a + 1, ns>([&](auto Q2) {
+          constexpr int b = decltype(Q2)::value;
+          constexpr int ib = Net::CPLX_ID[k][b];
+          constexpr double nab = na * Net::CPLX_NU[k][b];
+          if constexpr (ia == ib) D[ia] += (2.0 * nab) * mf;
+          else W[tri(ia, ib)] += nab * mf;
+        });
+      });
+    });
+  }
+  {
+    double* pt = A.total + c;
+    sfor<0, NAQ>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      const double total = (x[i] + tot[i]) * dkl;
+      *pt = total;
+      pt += ld;
+      res[i] = wet ? (psv * total - psv * fx[i]) / A.dt : 0.0;
+    });
+  }
+  double dimm[NI1];
+  sfor<0, NIMM>([&](auto I) {
+    constexpr int i = decltype(I)::value;
+    double r = (x[NAQ + i] * vol - fx[NAQ + i] * vol) / A.dt, d = vol / A.dt;
+    sfor<0, Net::NDECAY>([&](auto Dq) {
+      constexpr int q = decltype(Dq)::value;
+      if constexpr (Net::DECAY_ID[q] == i) {
+        const double kc = Net::DECAY_K[q] * vol;
+        r += kc * x[NAQ + i];
+        d += kc;
+      }
+    });
+    res[NAQ + i] = wet ? r : 0.0;
+    dimm[i] = wet ? d : 1.0;
+  });
+  sfor<0, NM>([&](auto Mq) {
+    constexpr int m = decltype(Mq)::value;
+    constexpr int ns = Net::MNRL_N[m];
+    double rt = 0.0;
+    if (wet && ar[m] != 0.0) {
+      const double QK = mnrl_q<m>(act, lnT, tk, ln_aw);
+      const MRate r = mineral_rate<m>(QK, vf[m], ar[m], temp);
+      if (r.active) {
+        rt = r.Im;
+        const double Iv = r.Im * vol, gm = r.dIm * vol * QK * dkl;
+        sfor<0, ns>([&](auto Q) {
+          constexpr int a = decltype(Q)::value;
+          constexpr int ia = Net::MNRL_ID[m][a];
+          constexpr double na = Net::MNRL_NU[m][a];
+          res[ia] += na * Iv;
+          D[ia] += (na * na) * gm;
+          sfor<a + 1, ns>([&](auto Q2) {
+            constexpr int b = decltype(Q2)::value;
+            constexpr int ib = Net::MNRL_ID[m][b];
+            constexpr double nab = na * Net::MNRL_NU[m][b];
+            if constexpr (ia == ib) D[ia] += (2.0 * nab) * gm;
+            else W[tri(ia, ib)] += nab * gm;
+          });
+        });
+      }
+    }
+    if (A.mnrl_rate) A.mnrl_rate[m * ld + c] = rt;
+  });
+  {
+    double* pr = A.res + c;
+    sfor<0, N>([&](auto I) {
+      *pr = res[decltype(I)::value];
+      pr += ld;
+    });
+  }
+  if (A.jac) {
+    double* pj = A.jac + c;
+    sfor<0, N>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      sfor<0, N>([&](auto J) {
+        constexpr int j = decltype(J)::value;
+        double v = 0.0;
+        if constexpr (i < NAQ && j < NAQ) {
+          if constexpr (i == j) v = wet ? D[i] * xi[i] + f : 1.0;
+          else v = wet ? W[tri(i, j)] * xi[j] : 0.0;
+        } else if constexpr (i == j) {
+          v = dimm[i - NAQ];
+        }
+        *pj = v;
+        pj += ld;
+      });
+    });
+  }
+}
+
+}  // namespace pflane
+
+#ifdef PFLANE_GIRT
+extern "C" __global__ void __launch_bounds__(64) pfchem_lane_girt(pflane::GirtArgs a) {
+  pflane::lane_girt(a);
 }
 #endif

@@ -230,8 +230,10 @@ class Context:
         s = st.to_abi()
         sp = (stream or torch.cuda.current_stream()).cuda_stream
         ncomp = self.net.naqcomp + self.net.nimmobile
-        res = torch.zeros((ncomp, st.ld), dtype=torch.float64, device="cuda")
-        jac = (torch.zeros((ncomp * ncomp, st.ld), dtype=torch.float64, device="cuda")
+        # the call writes every row of every cell; cells beyond ncell stay zero
+        new = torch.empty if st.ncell == st.ld else torch.zeros
+        res = new((ncomp, st.ld), dtype=torch.float64, device="cuda")
+        jac = (new((ncomp * ncomp, st.ld), dtype=torch.float64, device="cuda")
                if jacobian else None)
 
         def ptr(t):
