@@ -1385,7 +1385,7 @@ int sens_stage(pfchem_ctx* ctx, const double* wv, const double* ws, const double
   if (!ctx->sens_in) {
     if (hipMalloc(&ctx->sens_in, nin * sizeof(double)) != hipSuccess ||
         hipHostMalloc(&ctx->sens_in_h, nin * sizeof(double)) != hipSuccess ||
-        hipMalloc(&ctx->sens_sum, (np + 1) * sizeof(double)) != hipSuccess ||
+        hipMalloc(&ctx->sens_sum, (np + 1) * (1 + kSensSlices) * sizeof(double)) != hipSuccess ||
         hipHostMalloc(&ctx->sens_sum_h, (np + 1) * sizeof(double)) != hipSuccess ||
         hipEventCreateWithFlags(&ctx->sens_copied, hipEventDisableTiming) != hipSuccess)
       return fail(ctx, PFCHEM_ERR_NOMEM, "sensitivity buffers");

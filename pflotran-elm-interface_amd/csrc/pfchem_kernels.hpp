@@ -97,7 +97,9 @@ hipError_t launch_buckets(const int32_t* nact, int64_t ncell, int naq, int32_t* 
                           int32_t* counts, hipStream_t stream);
 
 // sensitivities (tangent: mode 0, out = df per cell; adjoint: mode 1, out =
-// per-cell gradients [q * ldo + cell], sum = their sum over converged cells)
+// per-cell gradients [q * ldo + cell], sum = their sum over converged cells,
+// followed by kSensSlices doubles of work space per parameter)
+constexpr int kSensSlices = 64;
 int sens_supported(const DevNet& n, const pfchem_options& opt);
 hipError_t launch_sens(const DevNet& n, const DevNet* dn, const DevState* ds, int64_t ncell,
                        double dt, const double* wv, const double* ws, const double* dp, int mode,

@@ -1871,18 +1871,28 @@ __device__ inline void lane_adjoint(const SensArgs& A) {
     bool cons = true;
     {
       double g0[NG1];
-      sfor<0, NC>([&](auto K) {
-        constexpr int k = decltype(K)::value;
-        constexpr int q = Net::CPLX_GCLS[k];
-        const double g = A.sec_act_coef[k * ld + c];
-        if constexpr (q < 0) {
-          cons = cons && g == 1.0;
-        } else if constexpr (Net::CPLX_GFIRST[k]) {
-          g0[q] = g;
-          gi[q] = 1.0 / g;
-        } else {
-          cons = cons && g == g0[q];
-        }
+      const double* pg = A.sec_act_coef + c;
+      constexpr int CH = 20;  // loads issued before the first is compared
+      sfor<0, (NC + CH - 1) / CH>([&](auto B) {
+        constexpr int k0 = decltype(B)::value * CH, k1 = k0 + CH < NC ? k0 + CH : NC;
+        double g[CH];
+        sfor<k0, k1>([&](auto K) {
+          g[decltype(K)::value - k0] = *pg;
+          pg += ld;
+        });
+        issue_loads();
+        sfor<k0, k1>([&](auto K) {
+          constexpr int k = decltype(K)::value;
+          constexpr int q = Net::CPLX_GCLS[k];
+          if constexpr (q < 0) {
+            cons &= g[k - k0] == 1.0;
+          } else if constexpr (Net::CPLX_GFIRST[k]) {
+            g0[q] = g[k - k0];
+            gi[q] = 1.0 / g[k - k0];
+          } else {
+            cons &= g[k - k0] == g0[q];
+          }
+        });
       });
     }
     if (!cons) {

@@ -503,22 +503,39 @@ sens_kernel(const DevNet* np, const DevState* sp, int64_t ncell, double dt,
 }
 
 // deterministic sum over cells of each parameter row of the per-cell
-// gradients (cells whose status is not 0 are skipped)
+// gradients (cells whose status is not 0 are skipped), in two launches: a
+// row's kSensSlices slices of consecutive cells, then the slices.  One
+// workgroup a row left the chip idle (65 rows of 131,072 cells: 356 us for
+// 68 MB; kRedTime in slices).
 __global__ void __launch_bounds__(256)
-sens_reduce_kernel(const double* __restrict__ g, int64_t ldo, int64_t ncell,
-                   const int32_t* __restrict__ status, double* __restrict__ sum) {
+sens_slice_kernel(const double* __restrict__ g, int64_t ldo, int64_t ncell,
+                  const int32_t* __restrict__ status, double* __restrict__ slices) {
   __shared__ double part[256];
-  const int q = blockIdx.x;
+  const int q = blockIdx.y;
+  const int64_t len = (ncell + kSensSlices - 1) / kSensSlices;
+  const int64_t c0 = blockIdx.x * len, c1 = c0 + len < ncell ? c0 + len : ncell;
   double acc = 0.0;
-  for (int64_t c = threadIdx.x; c < ncell; c += 256)
-    if (gld(status + c) == 0) acc += gld(g + q * ldo + c);
+  for (int64_t c = c0 + threadIdx.x; c < c1; c += 256)
+    if (status[c] == 0) acc += g[q * ldo + c];
   part[threadIdx.x] = acc;
   __syncthreads();
   for (int h = 128; h > 0; h >>= 1) {
     if ((int)threadIdx.x < h) part[threadIdx.x] += part[threadIdx.x + h];
     __syncthreads();
   }
-  if (threadIdx.x == 0) gst(sum + q, part[0]);
+  if (threadIdx.x == 0) slices[q * kSensSlices + blockIdx.x] = part[0];
+}
+__global__ void __launch_bounds__(kSensSlices)
+sens_reduce_kernel(const double* __restrict__ slices, double* __restrict__ sum) {
+  __shared__ double part[kSensSlices];
+  const int q = blockIdx.x;
+  part[threadIdx.x] = slices[q * kSensSlices + threadIdx.x];
+  __syncthreads();
+  for (int h = kSensSlices / 2; h > 0; h >>= 1) {
+    if ((int)threadIdx.x < h) part[threadIdx.x] += part[threadIdx.x + h];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) sum[q] = part[0];
 }
 
 }  // namespace
@@ -552,8 +569,11 @@ hipError_t launch_sens(const DevNet& n, const DevNet* dn, const DevState* ds, in
 #undef PFCHEM_SENS
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || mode != 1 || !sum) return e;
-  sens_reduce_kernel<<<dim3((unsigned)(n.nm + n.nc)), dim3(256), 0, stream>>>(out, ldo, ncell,
-                                                                               status, sum);
+  const unsigned np = (unsigned)(n.nm + n.nc);
+  double* slices = sum + np;
+  sens_slice_kernel<<<dim3(kSensSlices, np), dim3(256), 0, stream>>>(out, ldo, ncell, status,
+                                                                     slices);
+  sens_reduce_kernel<<<dim3(np), dim3(kSensSlices), 0, stream>>>(slices, sum);
   return hipGetLastError();
 }
 
