@@ -385,7 +385,8 @@ int pfchem_residual(pfchem_ctx* ctx, int64_t ncell, const pfchem_state* state,
    adds into the cell's diagonal block (reactive_transport.F90:3177, 3288).
    jac may be NULL.  Replaces the per-cell loop bodies of RTResidualNonFlux
    (reactive_transport.F90:2393-2430, 2599-2642) and RTJacobianNonFlux
-   (:3172-3183, 3270-3300) for a batch of cells. */
+   (:3172-3183, 3270-3300) for a batch of cells.  The first call of a network
+   that the one-lane kernel takes compiles its module. */
 int pfchem_residual_jacobian(pfchem_ctx* ctx, int64_t ncell, const pfchem_state* state,
                              const double* fixed_total, const double* fixed_immobile,
                              double dt, double* res, double* jac, void* stream);
@@ -396,6 +397,10 @@ int pfchem_residual_jacobian(pfchem_ctx* ctx, int64_t ncell, const pfchem_state*
    the device at the first batched step; it takes aqueous networks of up to
    16 primaries (plus immobile species with first-order decay) without the
    SomDec sandbox or per-cell active counts, and is then the default.
+   A SomDec network without complexes, minerals, an oxygen response and O2
+   tracking runs it too until a shape is set for the variant; the launch
+   reported for it is then the team shape of the cells that kernel hands
+   over.
    block_size must be 256 and blocks_per_cu caps the workgroups per CU (0:
    as many as its register use allows).  lanes_per_cell > 1: a team of
    lanes_per_cell lanes owns one cell (64 / lanes_per_cell cells per

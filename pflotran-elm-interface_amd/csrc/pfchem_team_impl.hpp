@@ -604,13 +604,6 @@ team_step_kernel(const DevNet* np, const DevState* sp, int64_t ncell, double dt,
     // rather than a few waves running the whole list several cells deep
     const int64_t waves = (int64_t)gridDim.x * (blockDim.x / 64);
     if (nwork < 4 * (int64_t)batch * waves) batch = 64 / L;
-    // fewer cells than wavefronts: one cell per wavefront, whose iteration is
-    // shorter without other teams' branches (the pass takes as long as its
-    // slowest cell)
-    if (nwork <= waves) {
-      batch = 1;
-      if (team_in_wave != 0) exhausted = true;
-    }
   }
 
   for (;;) {
