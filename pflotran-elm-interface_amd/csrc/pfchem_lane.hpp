@@ -2341,7 +2341,8 @@ __device__ inline void lane_girt(const GirtArgs& A) {
   // every load first
   const double por = A.porosity[c], sat = A.saturation[c], den = A.den_kg[c], vol = A.volume[c];
   const double temp = A.temperature ? A.temperature[c] : 25.0;
-  const double ln_aw = (Net::ACT_H2O && A.ln_act_h2o) ? A.ln_act_h2o[c] : 0.0;
+  // an input here, whether or not the option to update it is on
+  const double ln_aw = A.ln_act_h2o ? A.ln_act_h2o[c] : 0.0;
   double x[N], gam[NA1], fx[N], vf[NM1], ar[NM1], g[NC1];
   {
     const double* pp = A.pri_molal + c;

@@ -100,3 +100,46 @@ def run_host_adjoint(exe, net, state, dt, wv, ws, exact=True):
         f = np.fromfile(os.path.join(d, "fcell.out"), dtype=np.float64)
         st = np.fromfile(os.path.join(d, "status.out"), dtype=np.int32)
     return g[:npar], f, st
+
+
+def build_host_girt(net, opt, workdir):
+    """the generated residual and Jacobian block (PFLANE_GIRT) compiled for
+    the host"""
+    src = os.path.join(workdir, "lane_dev.hip")
+    rc = lib.prepare_kernels(net, opt, src)
+    assert rc == 0, "one-lane kernel does not take this network"
+    with open(src) as f:
+        text = f.read()
+    cpp = os.path.join(workdir, "lane_girt.cpp")
+    with open(cpp, "w") as f:
+        f.write("#define PFLANE_GIRT 1\n")
+        f.write(text)
+        f.write('\n#include "lane_host_girt.cpp"\n')
+    exe = os.path.join(workdir, "lane_host_girt")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-ffp-contract=off", "-w", "-I", HOST_DIR,
+                    "-include", os.path.join(HOST_DIR, "lane_host_shim.h"), cpp, "-o", exe],
+                   check=True)
+    return exe
+
+
+def run_host_girt(exe, net, state, fixed_total, fixed_imm, dt):
+    """(residual [ncomp, ncell], Jacobian [ncomp, ncomp, ncell], state with the
+    totals, secondary molalities and rates written back)"""
+    out = state.copy()
+    n, ncomp = state.ncell, net.naqcomp + net.nimmobile
+    with tempfile.TemporaryDirectory() as d:
+        for name in FIELDS:
+            a = out.arrays.get(name)
+            if a is not None and a.shape[0] > 0:
+                np.ascontiguousarray(a).tofile(os.path.join(d, name + ".bin"))
+        np.ascontiguousarray(fixed_total).tofile(os.path.join(d, "fixed_total.bin"))
+        if fixed_imm is not None:
+            np.ascontiguousarray(fixed_imm).tofile(os.path.join(d, "fixed_imm.bin"))
+        subprocess.run([exe, d, str(n), str(state.ld), repr(float(dt)), str(ncomp)], check=True)
+        res = np.fromfile(os.path.join(d, "res.out")).reshape(ncomp, -1)[:, :n]
+        jac = np.fromfile(os.path.join(d, "jac.out")).reshape(ncomp, ncomp, -1)[:, :, :n]
+        for name in ("total", "sec_molal", "mnrl_rate"):
+            p = os.path.join(d, name + ".out")
+            if os.path.exists(p):
+                out.arrays[name][...] = np.fromfile(p).reshape(out.arrays[name].shape)
+    return res, jac, out
