@@ -473,8 +473,9 @@ int pfchem_tune_cache_query(const char* cache_path, const char* key, const char*
    time (pfchem_step compiles them on the device at its first batched call).
    PFCHEM_ERR_UNSUPPORTED: the one-lane kernel does not take this network
    (the team kernels run it).  source_path (optional) receives the generated
-   device source.  No reference counterpart: the reference interprets the
-   network at run time (reaction_aux.F90:123-311). */
+   device source.  Takes the SomDec networks the one-lane step takes (see
+   pfchem_launch) too.  No reference counterpart: the reference interprets
+   the network at run time (reaction_aux.F90:123-311). */
 int pfchem_prepare_kernels(const pfchem_network* net, const pfchem_options* opt,
                            const char* source_path);
 

@@ -1275,7 +1275,13 @@ int pfchem_prepare_kernels(const pfchem_network* net, const pfchem_options* opt,
       !net->primary_spec_Z || !net->primary_spec_a0)
     return PFCHEM_ERR_INVALID;
   std::string why;
-  if (!lane_supported(net, opt, why)) return PFCHEM_ERR_UNSUPPORTED;
+  if (net->somdec) {
+    const int rc = check_somdec(net, why);
+    if (rc) return rc;
+    if (!lane_sd_supported(net, opt)) return PFCHEM_ERR_UNSUPPORTED;
+  } else if (!lane_supported(net, opt, why)) {
+    return PFCHEM_ERR_UNSUPPORTED;
+  }
   const std::string src = lane_source(net, opt);
   if (source_path) {
     FILE* f = std::fopen(source_path, "w");

@@ -37,15 +37,18 @@ int main(int argc, char** argv) {
   const char* names[] = {"pri_molal", "total", "immobile", "sec_molal", "pri_act_coef",
                          "sec_act_coef", "ln_act_h2o", "mnrl_volfrac", "mnrl_area", "mnrl_rate",
                          "porosity", "saturation", "den_kg", "volume", "temperature",
-                         "num_iterations", "num_sub_steps", "status"};
-  std::vector<std::vector<char>> buf(18);
+                         "num_iterations", "num_sub_steps", "status", "somdec_f_t",
+                         "somdec_f_w"};
+  constexpr int kFields = 20;
+  std::vector<std::vector<char>> buf(kFields);
   void** slots[] = {(void**)&a.pri_molal, (void**)&a.total, (void**)&a.immobile,
                     (void**)&a.sec_molal, (void**)&a.pri_act_coef, (void**)&a.sec_act_coef,
                     (void**)&a.ln_act_h2o, (void**)&a.mnrl_volfrac, (void**)&a.mnrl_area,
                     (void**)&a.mnrl_rate, (void**)&a.porosity, (void**)&a.saturation,
                     (void**)&a.den_kg, (void**)&a.volume, (void**)&a.temperature,
-                    (void**)&a.num_iterations, (void**)&a.num_sub_steps, (void**)&a.status};
-  for (int k = 0; k < 18; ++k) {
+                    (void**)&a.num_iterations, (void**)&a.num_sub_steps, (void**)&a.status,
+                    (void**)&a.sd_ft, (void**)&a.sd_fw};
+  for (int k = 0; k < kFields; ++k) {
     buf[k] = slurp(dir + "/" + names[k] + ".bin");
     *slots[k] = buf[k].empty() ? nullptr : (void*)buf[k].data();
   }
@@ -73,7 +76,7 @@ int main(int argc, char** argv) {
   } else {
     pfchem_lane_step_f64(a);
   }
-  for (int k = 0; k < 18; ++k)
+  for (int k = 0; k < kFields; ++k)
     if (!buf[k].empty()) spill(dir + "/" + names[k] + ".out", buf[k]);
   return 0;
 }

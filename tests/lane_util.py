@@ -19,7 +19,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 HOST_DIR = os.path.join(HERE, "lane_host")
 FIELDS = ("pri_molal", "total", "immobile", "sec_molal", "pri_act_coef", "sec_act_coef",
           "ln_act_h2o", "mnrl_volfrac", "mnrl_area", "mnrl_rate", "porosity", "saturation",
-          "den_kg", "volume", "temperature", "num_iterations", "num_sub_steps", "status")
+          "den_kg", "volume", "temperature", "num_iterations", "num_sub_steps", "status",
+          "somdec_f_t", "somdec_f_w")
 
 
 def build_host(net, opt, workdir):

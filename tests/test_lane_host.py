@@ -115,12 +115,14 @@ def test_rreact_call_bound(tmp_path):
 
 def test_prepare_refuses_other_networks():
     """the one-lane kernel takes aqueous networks of <= 16 primaries without
-    the sandbox, per-cell active counts or rate prefactors (whose Jacobian
-    terms are not symmetric); the others report UNSUPPORTED"""
+    per-cell active counts or rate prefactors (whose Jacobian terms are not
+    symmetric), and the sandbox without oxygen and complexes
+    (test_lane_host_somdec.py); the others report UNSUPPORTED"""
     wl = workloads.variable_network_workload(ncell=8)
     assert lib.prepare_kernels(wl.net, wl.opt) == abi.PFCHEM_ERR_UNSUPPORTED
-    wl = workloads.somdec_workload(ncell=8)
-    assert lib.prepare_kernels(wl.net, wl.opt) == abi.PFCHEM_ERR_UNSUPPORTED
+    for other in (dict(oxygen=1.0e-5), dict(complexes=True)):
+        wl = workloads.somdec_workload(ncell=8, **other)
+        assert lib.prepare_kernels(wl.net, wl.opt) == abi.PFCHEM_ERR_UNSUPPORTED
     import pin_util as PU
     wl = PU.prefactor_workload(8)
     assert lib.prepare_kernels(wl.net, wl.opt) == abi.PFCHEM_ERR_UNSUPPORTED
