@@ -438,7 +438,7 @@ __device__ __forceinline__ void sd_smooth(double c, double& H, double& dH) {
     if constexpr (x1 - x0 < 1.0e-50) {
       H = copysign(0.5, c - x1) + 0.5;
     } else {
-      constexpr double w = 1.0 / (x1 - x0);
+      constexpr double w = x1 > x0 ? 1.0 / (x1 - x0) : 0.0;  // formed for x0 = 0 too
       const double u = (c - x0) * w;
       const double xs = 1.0 - u * u;
       if (u < 0.0) {

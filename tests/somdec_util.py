@@ -20,7 +20,7 @@ def carbon_nitrogen(net, arrays, n):
 
 # networks that reach the sandbox's options the ELM-CN workload leaves unused
 OPTION_CASES = ("inhibition", "pool-monod", "responses", "scalars", "rates", "ammonium-only",
-                "smoothing", "linear", "no-split")
+                "smoothing", "no-smoothing", "linear", "no-split")
 
 
 def option_workload(which, ncell, seed=20261210):
@@ -78,6 +78,8 @@ def option_workload(which, ncell, seed=20261210):
         rx[0]["monod"], rx[1]["monod"] = mon[:1], []
     elif which == "smoothing":
         kw["x0eps"] = 1.0e-4
+    elif which == "no-smoothing":
+        kw["x0eps"] = 0.0
     elif which == "linear":
         opt = somdec_options(use_log_formulation=False)
     elif which == "no-split":
