@@ -27,9 +27,12 @@ const char kLaneTemplate[] =
 #include "pfchem_lane_src.inc"
     ;
 
-// exact decimal-free spelling of a double (C++17 hexadecimal literal)
+// exact decimal-free spelling of a double (C++17 hexadecimal literal); the
+// tables carry the caller's unused entries too, which may hold anything
 std::string hexd(double v) {
   char b[64];
+  if (std::isnan(v)) return "__builtin_nan(\"\")";
+  if (std::isinf(v)) return v > 0.0 ? "__builtin_inf()" : "-__builtin_inf()";
   if (v == 0.0) return std::signbit(v) ? "-0.0" : "0.0";
   std::snprintf(b, sizeof b, "%a", v);
   return b;

@@ -51,3 +51,24 @@ def test_somdec_options(which, tmp_path):
     for f32 in (False, True):
         got = LU.run_host(exe, wl.state, wl.dt, f32=f32)
         _compare(wl, ref, band, got, which + ("/mixed" if f32 else "/fp64"), 0.05)
+
+
+def test_unused_entries_of_the_descriptor(tmp_path):
+    """the per-reaction tables are as wide as the largest number of terms, and
+    a response's parameter is read by its own function only: whatever a caller
+    leaves in the unused entries, the kernel compiles and steps the same"""
+    wl = SU.option_workload("inhibition", 64)
+    exe = LU.build_host(wl.net, wl.opt, str(tmp_path))
+    want = LU.run_host(exe, wl.state, wl.dt)
+    a = wl.net.somdec.arrays
+    for name, count in (("monod_half_saturation", "n_monod"), ("monod_threshold", "n_monod"),
+                        ("inhibition_constant", "n_inhibition"),
+                        ("inhibition_constant2", "n_inhibition"),
+                        ("downstream_stoich", "n_downstream_pools")):
+        for r in range(wl.net.somdec.nrxn):
+            a[name][r, a[count][r]:] = (np.nan, np.inf, -np.inf)[r % 3]
+    a["Ea"][:], a["Q10"][:], a["Ox_half_saturation"][:] = np.nan, np.inf, np.nan
+    exe = LU.build_host(wl.net, wl.opt, str(tmp_path))
+    got = LU.run_host(exe, wl.state, wl.dt)
+    for f in ("status",) + FIELDS:
+        assert np.array_equal(got[f], want[f]), f
