@@ -422,6 +422,12 @@ __device__ __forceinline__ void sd_J(SdSum& s, double v) {
 }
 // dof of an immobile species (-1: none)
 constexpr int sd_row(int imm) { return imm >= 0 ? Net::NAQ + imm : -1; }
+// column p of the pattern has entries below the diagonal
+constexpr bool lu_eliminates(int p) {
+  for (int i = p + 1; i < Net::NAQ + Net::NIMM; ++i)
+    if (Net::JPOS[i][p] >= 0) return true;
+  return false;
+}
 __device__ __forceinline__ double sd_div(double a, double b) { return a * rcp_nr(b); }
 __device__ __forceinline__ double sd_monod(double c, double k) { return sd_div(c, c + k); }
 __device__ __forceinline__ double sd_dmonod(double c, double k) {
@@ -1434,7 +1440,14 @@ __device__ __forceinline__ void lane_step(const Args& A) {
       sfor<0, N>([&](auto P) {
         constexpr int p = decltype(P)::value;
         const JT pv = a[Net::JPOS[p][p]];
-        if (!((double)(pv < (JT)0 ? -pv : pv) > kLuTol * amax[p])) bad = true;
+        // A pivot small against its row makes the rows below it grow by its
+        // multipliers.  A column without entries below the diagonal has
+        // none: its unknown (a tracking species, the gases) is read off its
+        // own row, whose terms may be any multiple of the pivot, as they are
+        // where it starts empty.
+        const double av = (double)(pv < (JT)0 ? -pv : pv);
+        constexpr bool below = lu_eliminates(p);
+        if (!(av > (below ? kLuTol * amax[p] : 0.0) && av - av == 0.0)) bad = true;  // or not finite
         const JT inv = F32 ? (JT)1 / pv : (JT)rcp_nr((double)pv);
         pinv[p] = inv;
         sfor<p + 1, N>([&](auto Q) {

@@ -20,7 +20,7 @@ def carbon_nitrogen(net, arrays, n):
 
 # networks that reach the sandbox's options the ELM-CN workload leaves unused
 OPTION_CASES = ("inhibition", "pool-monod", "responses", "scalars", "rates", "ammonium-only",
-                "smoothing", "no-smoothing", "linear", "no-split")
+                "smoothing", "no-smoothing", "linear", "no-split", "trackers")
 
 
 def option_workload(which, ncell, seed=20261210):

@@ -2,7 +2,8 @@
 FP64 oracle over the sandbox's options: inhibition, pool-normalized Monod and
 thresholds, the temperature and moisture responses, the ELM scalars,
 decomposition rates, networks without nitrate, smoothing, the linear
-formulation and both forms of the NH4+ / NO3- split.
+formulation, both forms of the NH4+ / NO3- split, and tracking species that
+start empty (1e-20).
 
 Bar: that of test_gpu_somdec.py (the oracle's own spread under a ten-fold
 change of its convergence tolerances) on the cells that take the oracle's
