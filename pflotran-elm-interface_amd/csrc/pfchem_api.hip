@@ -82,6 +82,7 @@ struct pfchem_ctx {
   std::string lane_why;
   std::string lane_girt_src;  // the GIRT module's source (compiled at first use)
   bool lane_girt_ready = false;
+  bool lane_girt_off = false;  // its module did not compile: the team kernel runs the block
   std::string lane_adj_src;  // the adjoint module's source (compiled at first use)
   bool lane_adj_ready = false;
   LaunchCfg team_default{16, 1, 256, 4};  // team shape of the FP64 rescue pass
@@ -913,10 +914,22 @@ static bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
-static bool sd_lane_now(const pfchem_ctx* ctx, int64_t ncell, const DevState& d, hipStream_t s) {
+// the one-lane default of a SomDec network (no shape set); the module is
+// compiled here, and a network whose module does not compile keeps the team
+// kernel from then on
+static bool sd_lane_now(pfchem_ctx* ctx, int64_t ncell, const DevState& d, hipStream_t s) {
+  if (!ctx->sd_lane) return false;
   const bool ready = ctx->lane_ready && ncell <= ctx->esc_cap &&
                      (d.status || ncell <= ctx->status_cap);
-  return ctx->sd_lane && (ready || !capturing(s));
+  if (!ready && capturing(s)) return false;
+  if (!ctx->lane_ready) {
+    if (lane_compile(ctx->lane_src, ctx->device, ctx->lane_why)) {
+      ctx->sd_lane = false;
+      return false;
+    }
+    ctx->lane_ready = true;
+  }
+  return true;
 }
 static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double dt, bool mixed,
                      hipStream_t s) {
@@ -1172,18 +1185,17 @@ int pfchem_residual_jacobian(pfchem_ctx* ctx, int64_t ncell, const pfchem_state*
   hipError_t e = hipSetDevice(ctx->device);
   if (e != hipSuccess) return hip_fail(ctx, e, "hipSetDevice");
   hipStream_t s = (hipStream_t)stream;
-  if (ctx->lane_ok && (ctx->lane_girt_ready || !capturing(s))) {
-    // networks the one-lane kernel takes: a lane per cell, network constants
-    // compiled in (262,139 cells of the 15-primary network with the Jacobian:
-    // 286 us against 1,267 us of the team kernel; 0.84 GB, so 163 us at the
-    // rate of a copy)
-    if (!ctx->lane_girt_ready) {
-      ctx->lane_girt_src = std::string(kLaneGirtDefine) + ctx->lane_src;
-      std::string msg;
-      const int crc = lane_compile(ctx->lane_girt_src, ctx->device, msg);
-      if (crc) return fail(ctx, crc, msg);
-      ctx->lane_girt_ready = true;
-    }
+  // networks the one-lane kernel takes: a lane per cell, network constants
+  // compiled in (262,139 cells of the 15-primary network with the Jacobian:
+  // 286 us against 1,267 us of the team kernel; 0.84 GB, so 163 us at the
+  // rate of a copy).  A module that does not compile leaves the team kernel.
+  if (ctx->lane_ok && !ctx->lane_girt_ready && !ctx->lane_girt_off && !capturing(s)) {
+    ctx->lane_girt_src = std::string(kLaneGirtDefine) + ctx->lane_src;
+    std::string msg;
+    ctx->lane_girt_ready = lane_compile(ctx->lane_girt_src, ctx->device, msg) == PFCHEM_OK;
+    ctx->lane_girt_off = !ctx->lane_girt_ready;
+  }
+  if (ctx->lane_girt_ready) {
     LaneGirtArgs a{};
     a.ld = d.ld;
     a.ncell = ncell;
