@@ -901,27 +901,18 @@ static int to_dev_state(pfchem_ctx* ctx, const pfchem_state* st, int64_t ncell, 
   return PFCHEM_OK;
 }
 
-// Batched step on the network-specialized lane kernel: FP32 (mixed) or FP64
-// pass over every cell, then the FP64 team kernel (pivoting) over the cells
-// handed over.  The hand-over pass runs few cells, so its time is the
-// latency of its slowest cell: a team of lanes runs one Newton iteration
-// several times faster than one lane does.
-static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double dt, bool mixed,
-                     hipStream_t s);
-// a captured stream takes no module load and no allocation: a call whose
-// one-lane module or scratch is not there yet keeps the team kernel then
+// a captured stream takes no module load
 static bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
 // the one-lane default of a SomDec network (no shape set); the module is
 // compiled here, and a network whose module does not compile keeps the team
-// kernel from then on
-static bool sd_lane_now(pfchem_ctx* ctx, int64_t ncell, const DevState& d, hipStream_t s) {
-  if (!ctx->sd_lane) return false;
-  const bool ready = ctx->lane_ready && ncell <= ctx->esc_cap &&
-                     (d.status || ncell <= ctx->status_cap);
-  if (!ready && capturing(s)) return false;
+// kernel from then on.  A captured step keeps the team kernel: the one-lane
+// step waits for the event that guards its hand-over list, which was recorded
+// outside the capture, and a graph would hold that list past its regrowth.
+static bool sd_lane_now(pfchem_ctx* ctx, hipStream_t s) {
+  if (!ctx->sd_lane || capturing(s)) return false;
   if (!ctx->lane_ready) {
     if (lane_compile(ctx->lane_src, ctx->device, ctx->lane_why)) {
       ctx->sd_lane = false;
@@ -931,6 +922,12 @@ static bool sd_lane_now(pfchem_ctx* ctx, int64_t ncell, const DevState& d, hipSt
   }
   return true;
 }
+
+// Batched step on the network-specialized lane kernel: FP32 (mixed) or FP64
+// pass over every cell, then the FP64 team kernel (pivoting) over the cells
+// handed over.  The hand-over pass runs few cells, so its time is the
+// latency of its slowest cell: a team of lanes runs one Newton iteration
+// several times faster than one lane does.
 static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double dt, bool mixed,
                      hipStream_t s) {
   if (!ctx->lane_ok && !ctx->sd_lane)
@@ -1140,7 +1137,7 @@ int pfchem_step(pfchem_ctx* ctx, int64_t ncell, const pfchem_state* state, doubl
       return PFCHEM_OK;
     }
     const LaunchCfg& cfg = ctx->launch[variant];
-    if (cfg.lanes_per_cell == 1 || (!ctx->launch_set[variant] && sd_lane_now(ctx, ncell, d, s)))
+    if (cfg.lanes_per_cell == 1 || (!ctx->launch_set[variant] && sd_lane_now(ctx, s)))
       return lane_step(ctx, ncell, d, dt, mixed, s);
     if (!team_supports(ctx->dnet, cfg, mixed))
       return fail(ctx, PFCHEM_ERR_UNSUPPORTED, "launch configuration does not fit this network");
