@@ -398,9 +398,9 @@ int pfchem_residual_jacobian(pfchem_ctx* ctx, int64_t ncell, const pfchem_state*
    16 primaries (plus immobile species with first-order decay) without the
    SomDec sandbox or per-cell active counts, and is then the default.
    A SomDec network without complexes, minerals, an oxygen response and O2
-   tracking runs it too until a shape is set for the variant; the launch
-   reported for it is then the team shape of the cells that kernel hands
-   over.
+   tracking runs it by default too.  The launch reported for that default is
+   the team shape of the cells the kernel hands over, and setting that shape
+   restores the default; any other team shape runs the team kernel alone.
    block_size must be 256 and blocks_per_cu caps the workgroups per CU (0:
    as many as its register use allows).  lanes_per_cell > 1: a team of
    lanes_per_cell lanes owns one cell (64 / lanes_per_cell cells per

@@ -75,10 +75,12 @@ struct pfchem_ctx {
   std::string lane_src;
   bool lane_ok = false;
   bool lane_ready = false;
-  // a SomDec network the step kernel takes: it runs until a launch shape is
-  // set (launch holds the team shape of the pass over handed-over cells)
+  // a SomDec network the step kernel takes: it runs while the variant's shape
+  // is launch_default, the team shape of the pass over handed-over cells,
+  // which is how that default is named (get_launch reports it, and setting
+  // what was reported changes nothing)
   bool sd_lane = false;
-  bool launch_set[3] = {};
+  LaunchCfg launch_default[3] = {};
   std::string lane_why;
   std::string lane_girt_src;  // the GIRT module's source (compiled at first use)
   bool lane_girt_ready = false;
@@ -765,6 +767,8 @@ int pfchem_create(const pfchem_network* net, const pfchem_options* opt, int devi
       ctx->launch[v] = LaunchCfg{1, 1, 256, 0, ctx->max_lds};
   } else if (lane_sd_supported(net, opt)) {
     ctx->sd_lane = true;
+    for (int v = PFCHEM_KERNEL_BATCHED_FP64; v <= PFCHEM_KERNEL_BATCHED_MIXED; ++v)
+      ctx->launch_default[v] = ctx->launch[v];
     ctx->lane_src = lane_source(net, opt);
   }
   if (hipMalloc(&ctx->dnet_dev, sizeof(DevNet)) != hipSuccess ||
@@ -906,13 +910,17 @@ static bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
-// the one-lane default of a SomDec network (no shape set); the module is
+// the one-lane default of a SomDec network; the module is
 // compiled here, and a network whose module does not compile keeps the team
 // kernel from then on.  A captured step keeps the team kernel: the one-lane
 // step waits for the event that guards its hand-over list, which was recorded
 // outside the capture, and a graph would hold that list past its regrowth.
-static bool sd_lane_now(pfchem_ctx* ctx, hipStream_t s) {
-  if (!ctx->sd_lane || capturing(s)) return false;
+static bool sd_lane_now(pfchem_ctx* ctx, int variant, hipStream_t s) {
+  const LaunchCfg &c = ctx->launch[variant], &d = ctx->launch_default[variant];
+  if (!ctx->sd_lane || c.lanes_per_cell != d.lanes_per_cell ||
+      c.rows_per_lane != d.rows_per_lane || c.block_size != d.block_size ||
+      c.blocks_per_cu != d.blocks_per_cu || capturing(s))
+    return false;
   if (!ctx->lane_ready) {
     if (lane_compile(ctx->lane_src, ctx->device, ctx->lane_why)) {
       ctx->sd_lane = false;
@@ -1137,7 +1145,7 @@ int pfchem_step(pfchem_ctx* ctx, int64_t ncell, const pfchem_state* state, doubl
       return PFCHEM_OK;
     }
     const LaunchCfg& cfg = ctx->launch[variant];
-    if (cfg.lanes_per_cell == 1 || (!ctx->launch_set[variant] && sd_lane_now(ctx, s)))
+    if (cfg.lanes_per_cell == 1 || sd_lane_now(ctx, variant, s))
       return lane_step(ctx, ncell, d, dt, mixed, s);
     if (!team_supports(ctx->dnet, cfg, mixed))
       return fail(ctx, PFCHEM_ERR_UNSUPPORTED, "launch configuration does not fit this network");
@@ -1259,14 +1267,12 @@ int pfchem_set_launch(pfchem_ctx* ctx, int variant, const pfchem_launch* cfg) {
     if (c.rows_per_lane != 1 || c.block_size != 256)
       return fail(ctx, PFCHEM_ERR_INVALID, "the one-lane kernel runs 256-lane workgroups, 1 row");
     ctx->launch[variant] = c;
-    ctx->launch_set[variant] = true;
     return PFCHEM_OK;
   }
   if (variant != PFCHEM_KERNEL_PLAIN_FP64 &&
       !team_supports(ctx->dnet, c, variant == PFCHEM_KERNEL_BATCHED_MIXED))
     return fail(ctx, PFCHEM_ERR_UNSUPPORTED, "launch configuration does not fit this network");
   ctx->launch[variant] = c;
-  ctx->launch_set[variant] = true;
   if (ctx->dnet.variable && variant != PFCHEM_KERNEL_PLAIN_FP64 && c.rows_per_lane == 1)
     for (int b = 0; b < kBuckets; ++b)
       if (kBucketBound[b] == c.lanes_per_cell) ctx->vlaunch[variant - 1][b] = c;

@@ -48,3 +48,66 @@ def test_somdec_lane_and_team_agree(variant):
         # the iteration ends at 1e-8 relative change: one iteration more or
         # less moves an entry by at most that much of its row's range
         assert err.max() <= 1e-8, f
+
+
+def _one_lane(ctx, wl, variant):
+    """whether a step of this context ran the one-lane kernel (its pass is
+    what pfchem_set_pass_timing times)"""
+    import torch
+    from pfchem.lib import DeviceState, PfchemError
+    ctx.set_pass_timing(True)
+    ctx.step(DeviceState(wl.state), wl.dt, variant)
+    torch.cuda.synchronize()
+    try:
+        return ctx.pass_time() > 0.0
+    except PfchemError:
+        return False
+    finally:
+        ctx.set_pass_timing(False)
+
+
+@pytest.mark.parametrize("variant", VARIANTS)
+def test_reported_shape_restores_the_default(variant):
+    """reading and setting a shape changes no kernel, and the shape of a fresh
+    context brings its kernel back"""
+    from pfchem.lib import Context
+    wl = workloads.somdec_workload(300)
+    ctx = Context(wl.net, wl.opt)
+    start = ctx.get_launch(variant)
+    put = lambda l: ctx.set_launch(variant, l["lanes_per_cell"], l["block_size"],
+                                   l["blocks_per_cu"], l["rows_per_lane"])
+    assert _one_lane(ctx, wl, variant)
+    put(start)
+    assert ctx.get_launch(variant) == start and _one_lane(ctx, wl, variant)
+    for shape in ((8, 128, 4, 2), (16, 128, 4, 1), (1, 256, 1, 1)):
+        ctx.set_launch(variant, *shape)
+        assert _one_lane(ctx, wl, variant) == (shape[0] == 1)
+        kept = ctx.get_launch(variant)
+        put(kept)
+        assert ctx.get_launch(variant) == kept
+        assert _one_lane(ctx, wl, variant) == (shape[0] == 1)
+    put(start)
+    assert _one_lane(ctx, wl, variant)
+
+
+@pytest.mark.parametrize("variant", VARIANTS)
+def test_tuning_keeps_the_one_lane_step(variant, tmp_path):
+    """the tuner starts from the default kernel, leaves the state as given and
+    ends on a shape that still runs it (the teams are several times slower
+    here); so does a context that applies its cache"""
+    import torch
+    from pfchem.lib import Context, DeviceState
+    wl = workloads.somdec_workload(60000)
+    ctx = Context(wl.net, wl.opt)
+    ds = DeviceState(wl.state)
+    cache = str(tmp_path / "tune.json")
+    ctx.autotune(ds, wl.dt, variant, cache_path=cache, quick=True)
+    torch.cuda.synchronize()
+    back = ds.to_host()
+    for f in FIELDS:
+        assert np.array_equal(back[f], wl.state[f]), f
+    small = workloads.somdec_workload(300)
+    assert _one_lane(ctx, small, variant)
+    other = Context(wl.net, wl.opt)
+    other.autotune(ds, wl.dt, variant, cache_path=cache)  # the cached choice
+    assert _one_lane(other, small, variant)
