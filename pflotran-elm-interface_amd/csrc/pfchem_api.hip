@@ -807,13 +807,16 @@ TuneInfo tune_info(const pfchem_ctx* ctx) {
   t.lane_ok = ctx->lane_ok || ctx->sd_lane;
   int p2 = 1;
   while (p2 < d.ncomp) p2 *= 2;
+  // SomDec: 1 the team kernels alone, 2 the one-lane kernel too.  A team shape
+  // recorded for the first, or before the second existed, is no choice for it.
+  const int sd = ctx->sd_lane ? 2 : ctx->has_somdec ? 1 : 0;
   char buf[256];
   std::snprintf(buf, sizeof(buf), "%s/%dcu/aq%d/im%d/cx%d/mn%d/sd%d/var%d/%016llx",
                 ctx->arch.c_str(), ctx->num_cus, t.naq, t.nimm, t.neqcplx, t.nkinmnrl,
-                ctx->has_somdec ? 1 : 0, t.variable ? 1 : 0, (unsigned long long)ctx->net_hash);
+                sd, t.variable ? 1 : 0, (unsigned long long)ctx->net_hash);
   t.key = buf;
   std::snprintf(buf, sizeof(buf), "%s/%dcu/n%d/sd%d/var%d/lane%d", ctx->arch.c_str(),
-                ctx->num_cus, p2, ctx->has_somdec ? 1 : 0, t.variable ? 1 : 0,
+                ctx->num_cus, p2, sd, t.variable ? 1 : 0,
                 ctx->lane_ok ? 1 : 0);
   t.bucket = buf;
   if (t.variable) {

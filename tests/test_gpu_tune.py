@@ -101,3 +101,32 @@ def test_autotune_per_cell_active_counts(tmp_path):
         e = float(G.rel_err(got[f][:, :n], ref[f][:, :n]).max())
         print("tuned variable", f, e, flush=True)
         assert e <= CONC_TOL, (f, e)
+
+
+def test_somdec_kernel_families_share_no_cache_entry(tmp_path):
+    """a SomDec network the one-lane kernel takes applies no team shape that
+    was recorded for a network it refuses (oxygen), nor one recorded for the
+    same network under the key it had without the kernel"""
+    wl = workloads.somdec_workload(64)
+    ox = workloads.somdec_workload(64, oxygen=1.0e-5)
+    ctx = Context(wl.net, wl.opt)
+    start = ctx.get_launch(abi.KERNEL_BATCHED_FP64)
+    (key, bucket), (oxkey, oxbucket) = ctx.tune_key(), Context(ox.net, ox.opt).tune_key()
+    assert bucket != oxbucket
+    plain = lambda s: s.replace("/sd2/", "/sd1/")
+    assert plain(key) != key and plain(bucket) == oxbucket
+    cache = str(tmp_path / "tune.json")
+
+    def write(key, bucket):
+        e = {"key": key, "bucket": bucket, "variant": abi.KERNEL_BATCHED_FP64, "size_bucket": -1,
+             "ncell": 1 << 16, "lanes_per_cell": 8, "rows_per_lane": 2, "block_size": 128,
+             "blocks_per_cu": 4, "ms": 1.0, "default_ms": 2.0}
+        with open(cache, "w") as f:
+            f.write('{"pfchem_tune_cache": 1, "entries": [\n%s\n]}\n' % json.dumps(e))
+
+    for k, b in ((oxkey, oxbucket), (plain(key), plain(bucket))):
+        write(k, b)
+        assert _tuned_context_from_env(wl, cache).get_launch(abi.KERNEL_BATCHED_FP64) == start
+    write(key, bucket)  # its own entry applies
+    got = _tuned_context_from_env(wl, cache).get_launch(abi.KERNEL_BATCHED_FP64)
+    assert (got["lanes_per_cell"], got["rows_per_lane"]) == (8, 2)
