@@ -120,9 +120,23 @@ constexpr int kProdMinAq = 9;
 
 // 1 if the lane kernel handles this network and these options (else `why`)
 int lane_supported(const pfchem_network* net, const pfchem_options* opt, std::string& why);
+// Entries of the SomDec Jacobian pattern up to which the step kernel takes a
+// network.  Its unrolled elimination grows with the pattern, and with it the
+// first step's compile and the FP64 kernel's scratch.  200,000 cells, one step
+// of the default against the team kernel alone, FP64 and mixed:
+//   entries  unknowns  compile  scratch    FP64 ms        mixed ms
+//   115      15        2.2 s    144 B      26.3 / 34.2    26.5 / 38.8
+//   181      24        5.2 s    976 B      63.4 / 216     64.0 / 396
+//   271      22        6.9 s    1,856 B    38.4 / 49.1    38.7 / 74.6
+//   389      26        17.8 s   3,920 B    29.6 / 45.4    21.5 / 59.7
+// (most of the default's time is the handed-over cells').  Beyond 288 the
+// compile grows faster than the pattern (528 entries: 2-3 times the 389 ones)
+// for what a step gains, so larger networks keep the team kernel, which
+// compiles nothing.
+constexpr int kSdMaxEntries = 288;
 // 1 if the step kernel takes this network with its SomDec sandbox (no
 // complexes, minerals, Monod oxygen response, O2 tracking or activity update
-// per Newton iteration)
+// per Newton iteration, at most kSdMaxEntries pattern entries)
 int lane_sd_supported(const pfchem_network* net, const pfchem_options* opt);
 // full device source: the network as constants followed by the template
 std::string lane_source(const pfchem_network* net, const pfchem_options* opt);

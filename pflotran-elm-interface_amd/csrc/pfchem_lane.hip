@@ -203,6 +203,57 @@ int lane_supported(const pfchem_network* net, const pfchem_options* opt, std::st
   return 1;
 }
 
+namespace {
+// The sandbox's Jacobian pattern: every entry pfchem_lane.hpp adds, the
+// diagonal, and the fill-in of the elimination in natural order.  pos[row][col]
+// numbers the entries (-1: none); returns their count.
+int sd_pattern(const pfchem_network* net, std::vector<std::vector<int>>& pos) {
+  const pfchem_somdec* sd = net->somdec;
+  const int naq = net->naqcomp, N = naq + net->nimmobile, nr = sd->nrxn;
+  const int MD = PFCHEM_SOMDEC_MAX_DOWN;
+  pos.assign(N, std::vector<int>(N, -1));
+  auto put = [&](int row, int col) {
+    if (row >= 0 && col >= 0) pos[row][col] = 0;
+  };
+  auto dof = [&](int imm) { return imm >= 0 ? naq + imm : -1; };
+  for (int i = 0; i < N; ++i) put(i, i);
+  const int nh4 = sd->species_id_nh4, no3 = sd->species_id_no3;
+  for (int r = 0; r < nr; ++r) {
+    const bool vary = sd->upstream_is_varycn[r] != 0;
+    const int uc = dof(sd->upstream_c_id[r]);
+    for (int col : {uc, nh4, no3}) {
+      if (col != uc && !(vary || sd->mineral_n_stoich[r] < 0.0)) continue;
+      if (col == uc || sd->species_id_co2 == col) put(sd->species_id_co2, col);
+      put(uc, col);
+      put(dof(sd->upstream_hr_id[r]), col);
+      put(dof(sd->species_id_hr), col);
+      if (col == uc) put(nh4, col), put(no3, col);
+      put(dof(sd->upstream_nmin_id[r]), col);
+      put(dof(sd->species_id_nmin), col);
+      put(dof(sd->upstream_nimm_id[r]), col);
+      put(dof(sd->species_id_nimm), col);
+      if (vary) put(dof(sd->upstream_n_id[r]), col);
+      for (int j = 0; j < sd->n_downstream_pools[r]; ++j) {
+        put(dof(sd->downstream_c_id[r * MD + j]), col);
+        if (sd->downstream_is_varycn[r * MD + j]) put(dof(sd->downstream_n_id[r * MD + j]), col);
+      }
+    }
+  }
+  if (sd->species_id_n2o >= 0) put(dof(sd->species_id_ngasmin), nh4);
+  for (int p = 0; p < N; ++p)
+    for (int i = p + 1; i < N; ++i)
+      if (pos[i][p] >= 0)
+        for (int j = p + 1; j < N; ++j)
+          if (pos[p][j] >= 0) pos[i][j] = 0;
+  int nnz = 0;
+  for (auto& row : pos)
+    for (int& q : row)
+      if (q >= 0) q = nnz++;
+  return nnz;
+}
+
+}  // namespace
+
 int lane_sd_supported(const pfchem_network* net, const pfchem_options* opt) {
   const pfchem_somdec* sd = net->somdec;
   const int naq = net->naqcomp, nimm = net->nimmobile;
@@ -213,12 +264,11 @@ int lane_sd_supported(const pfchem_network* net, const pfchem_options* opt) {
   if (sd->species_id_co2 < 0 || sd->species_id_nh4 < 0 || sd->species_o2 != 0) return 0;
   for (int r = 0; r < sd->nrxn; ++r)
     if (sd->Ox_response_function[r] == 1) return 0;
-  return 1;
+  std::vector<std::vector<int>> pos;
+  return sd_pattern(net, pos) <= kSdMaxEntries;
 }
 
-// the sandbox's constants and its Jacobian pattern: every entry
-// pfchem_lane.hpp adds, the diagonal, and the fill-in of the elimination in
-// natural order
+// the sandbox's constants and its Jacobian pattern
 static void sd_source(Gen& g, const pfchem_network* net) {
   const pfchem_somdec* sd = net->somdec;
   const int naq = net->naqcomp, N = naq + net->nimmobile, nr = sd->nrxn;
@@ -308,44 +358,8 @@ static void sd_source(Gen& g, const pfchem_network* net) {
   g.ivec("SD_TCLS", tc);
   g.ivec("SD_WCLS", wc);
   // Jacobian pattern
-  std::vector<std::vector<int>> pos(N, std::vector<int>(N, -1));
-  auto put = [&](int row, int col) {
-    if (row >= 0 && col >= 0) pos[row][col] = 0;
-  };
-  auto dof = [&](int imm) { return imm >= 0 ? naq + imm : -1; };
-  for (int i = 0; i < N; ++i) put(i, i);
-  const int nh4 = sd->species_id_nh4, no3 = sd->species_id_no3;
-  for (int r = 0; r < nr; ++r) {
-    const bool vary = sd->upstream_is_varycn[r] != 0;
-    const int uc = dof(sd->upstream_c_id[r]);
-    for (int col : {uc, nh4, no3}) {
-      if (col != uc && !(vary || sd->mineral_n_stoich[r] < 0.0)) continue;
-      if (col == uc || sd->species_id_co2 == col) put(sd->species_id_co2, col);
-      put(uc, col);
-      put(dof(sd->upstream_hr_id[r]), col);
-      put(dof(sd->species_id_hr), col);
-      if (col == uc) put(nh4, col), put(no3, col);
-      put(dof(sd->upstream_nmin_id[r]), col);
-      put(dof(sd->species_id_nmin), col);
-      put(dof(sd->upstream_nimm_id[r]), col);
-      put(dof(sd->species_id_nimm), col);
-      if (vary) put(dof(sd->upstream_n_id[r]), col);
-      for (int j = 0; j < sd->n_downstream_pools[r]; ++j) {
-        put(dof(sd->downstream_c_id[r * MD + j]), col);
-        if (sd->downstream_is_varycn[r * MD + j]) put(dof(sd->downstream_n_id[r * MD + j]), col);
-      }
-    }
-  }
-  if (sd->species_id_n2o >= 0) put(dof(sd->species_id_ngasmin), nh4);
-  for (int p = 0; p < N; ++p)
-    for (int i = p + 1; i < N; ++i)
-      if (pos[i][p] >= 0)
-        for (int j = p + 1; j < N; ++j)
-          if (pos[p][j] >= 0) pos[i][j] = 0;
-  int nnz = 0;
-  for (auto& row : pos)
-    for (int& q : row)
-      if (q >= 0) q = nnz++;
+  std::vector<std::vector<int>> pos;
+  const int nnz = sd_pattern(net, pos);
   g.i("JNNZ", nnz);
   g.imat("JPOS", pos, N);
 }

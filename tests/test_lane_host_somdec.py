@@ -73,3 +73,31 @@ def test_unused_entries_of_the_descriptor(tmp_path):
     got = LU.run_host(exe, wl.state, wl.dt)
     for f in ("status",) + FIELDS:
         assert np.array_equal(got[f], want[f]), f
+
+
+def _cascade(nlit, nsom):
+    """litter pools of variable C:N onto a chain of SOM pools"""
+    from pfchem import somdec as SD
+    from pfchem.network import ReactionNetwork
+    prim = ["CO2(aq)", "NH4+", "NO3-", "N2O(aq)", "H+"]
+    imm = ["SOM%d" % i for i in range(nsom)]
+    imm += [n % i for i in range(nlit) for n in ("Lit%dC", "Lit%dN")]
+    mon = [SD.Monod("NH4+", 1e-6), SD.Monod("NO3-", 1e-6)]
+    rx = [SD.Reaction("Lit%d" % i, [("SOM%d" % (i % nsom), 0.5)], rate_constant=1e-6, monod=mon)
+          for i in range(nlit)]
+    rx += [SD.Reaction("SOM%d" % i, [("SOM%d" % (i + 1), 0.5)] if i + 1 < nsom else [],
+                       rate_constant=1e-7) for i in range(nsom)]
+    pools = [SD.Pool("SOM%d" % i, 12.0) for i in range(nsom)]
+    pools += [SD.Pool("Lit%d" % i) for i in range(nlit)]
+    return ReactionNetwork(primary_species_names=prim, primary_spec_Z=np.zeros(5),
+                           primary_spec_a0=np.zeros(5), immobile_names=imm,
+                           somdec=SD.build_somdec(pools, rx, prim, imm))
+
+
+@pytest.mark.parametrize("nlit,nsom,takes", [(3, 4, True), (6, 9, False), (7, 11, False)])
+def test_large_networks_keep_the_team_kernel(nlit, nsom, takes):
+    """networks whose unrolled elimination would take the first step long to
+    compile (389 and 528 pattern entries; 115 for the ELM-CN cascade's size)"""
+    from pfchem import abi, lib
+    want = abi.PFCHEM_OK if takes else abi.PFCHEM_ERR_UNSUPPORTED
+    assert lib.prepare_kernels(_cascade(nlit, nsom), workloads.somdec_options()) == want
