@@ -1197,7 +1197,8 @@ int pfchem_residual_jacobian(pfchem_ctx* ctx, int64_t ncell, const pfchem_state*
   // compiled in (262,139 cells of the 15-primary network with the Jacobian:
   // 286 us against 1,267 us of the team kernel; 0.84 GB, so 163 us at the
   // rate of a copy).  A module that does not compile leaves the team kernel.
-  if (ctx->lane_ok && !ctx->lane_girt_ready && !ctx->lane_girt_off && !capturing(s)) {
+  if (ctx->lane_ok && ctx->net.neqcplx <= kLaneGirtMaxCplx && !ctx->lane_girt_ready &&
+      !ctx->lane_girt_off && !capturing(s)) {
     ctx->lane_girt_src = std::string(kLaneGirtDefine) + ctx->lane_src;
     std::string msg;
     ctx->lane_girt_ready = lane_compile(ctx->lane_girt_src, ctx->device, msg) == PFCHEM_OK;

@@ -111,6 +111,14 @@ struct LaneGirtArgs {
   double dt;
 };
 static_assert(sizeof(LaneGirtArgs) == 176, "LaneGirtArgs layout");
+// Complexes up to which the GIRT block runs one cell per lane.  The kernel is
+// faster at every size (131,072 cells, 5 minerals, block against the team
+// kernel: 15 x 60 123 / 588 us, 16 x 100 155 / 809, 16 x 150 217 / 1,085,
+// 16 x 200 354 / 1,343), but its module is compiled in the first call, and it
+// holds a coefficient per complex: 1.8 s at 60, 5.7 s and 172 B of scratch at
+// 150, 9.5 s and 884 B at 200, 12.8 s at 250.  The line keeps the first call
+// under that of the largest SomDec step (7 s).
+constexpr int kLaneGirtMaxCplx = 160;
 // prefix of lane_source that makes a GIRT module
 constexpr char kLaneGirtDefine[] = "#define PFLANE_GIRT 1\n";
 

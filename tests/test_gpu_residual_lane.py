@@ -33,3 +33,33 @@ def test_residual_lane_edges(which, ncell, jacobian):
         assert jac is None
     np.testing.assert_allclose(got["total"][:, :ncell], t_ref, rtol=1e-13)
     np.testing.assert_allclose(got["sec_molal"][:, :ncell], s_ref, rtol=1e-13)
+
+
+@pytest.mark.parametrize("ncplx,one_lane", [(160, True), (161, False)])
+def test_residual_on_both_sides_of_the_size_line(ncplx, one_lane):
+    """networks of many complexes keep the team kernel, whose first call
+    compiles nothing (the module of the smaller one takes seconds)"""
+    import time
+    import torch
+    from pfchem import workloads
+    from pfchem.lib import Context, DeviceState
+    wl = workloads.random_network_workload(ncell=70, naq=16, ncplx=ncplx, nmnrl=5)
+    st = wl.state
+    fixed = st["total"][:16] * 1.001
+    r_ref, j_ref, t_ref, s_ref, acc = _oracle(wl, st, fixed, None, np.arange(70), DT)
+    ctx = Context(wl.net, wl.opt)
+    ds, fx = DeviceState(st), torch.from_numpy(np.ascontiguousarray(fixed)).cuda()
+    torch.cuda.synchronize()
+    t0 = time.perf_counter()
+    res, jac = ctx.residual(ds, fx, None, DT)
+    torch.cuda.synchronize()
+    first = time.perf_counter() - t0
+    print("first call %.2f s" % first, flush=True)
+    assert one_lane or first < 2.0
+    assert np.all(np.abs(res.cpu().numpy() - r_ref) <= 1e-9 * np.maximum(np.abs(r_ref), 1e-12 * acc))
+    j = jac.cpu().numpy().reshape(j_ref.shape)
+    scale = np.abs(j_ref).max(axis=1, keepdims=True)
+    assert (np.abs(j - j_ref) / np.where(scale > 0, scale, 1.0)).max() <= 1e-11
+    got = ds.to_host()
+    np.testing.assert_allclose(got["total"], t_ref, rtol=1e-13)
+    np.testing.assert_allclose(got["sec_molal"], s_ref, rtol=1e-13)
