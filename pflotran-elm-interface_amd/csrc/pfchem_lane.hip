@@ -521,10 +521,15 @@ std::string lane_source(const pfchem_network* net, const pfchem_options* opt) {
   return g.s;
 }
 
+// Compiling takes seconds: the lock that every launch of a module takes is not
+// held meanwhile.  Two threads may compile the same source; the first to
+// finish stores its module, the other drops its own.
 int lane_compile(const std::string& src, int device, std::string& err) {
-  std::lock_guard<std::mutex> lk(g_mu);
   const auto key = std::make_pair(device, src);
-  if (g_mods.count(key)) return PFCHEM_OK;
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    if (g_mods.count(key)) return PFCHEM_OK;
+  }
   std::vector<char> code;
   const int rc = lane_compile_only(src, &code, err);
   if (rc) return rc;
@@ -546,12 +551,14 @@ int lane_compile(const std::string& src, int device, std::string& err) {
       e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&m.blocks_per_cu64, m.f64, 256, 0);
   }
   if (e != hipSuccess) {
+    if (m.mod) (void)hipModuleUnload(m.mod);
     err = std::string("lane kernel load: ") + hipGetErrorString(e);
     return PFCHEM_ERR_HIP;
   }
   if (m.blocks_per_cu32 < 1) m.blocks_per_cu32 = 1;
   if (m.blocks_per_cu64 < 1) m.blocks_per_cu64 = 1;
-  g_mods[key] = m;
+  std::lock_guard<std::mutex> lk(g_mu);
+  if (!g_mods.emplace(key, m).second) (void)hipModuleUnload(m.mod);
   return PFCHEM_OK;
 }
 
