@@ -342,10 +342,11 @@ const char* pfchem_last_error(const pfchem_ctx* ctx);
    `stream` (a hipStream_t, NULL = default stream) and returns without
    synchronizing.  Per-cell outcome goes to state->status; the call itself
    returns PFCHEM_OK if the launch succeeded.  Calls on one context may use
-   different streams; steps that use the context's scratch lists (the
-   one-lane kernel's hand-over list, the status array kept when
-   state->status is NULL, the size buckets) run one after another on the
-   device, whatever their streams.
+   different streams.  The one-lane kernel's lists (handed-over cells, and the
+   status when state->status is NULL) are kept in four sets: steps on up to
+   four streams do not wait for each other, further streams share a set, and
+   steps that share one run one after another on the device, as do steps with
+   per-cell active counts (their size buckets).
    Replaces RStep (reaction.F90:3564) applied to every local cell. */
 int pfchem_step(pfchem_ctx* ctx, int64_t ncell, const pfchem_state* state,
                 double dt, int variant, void* stream);

@@ -18,6 +18,23 @@
 
 using namespace pfchem;
 
+// Lists of one one-lane step: the cells it hands over and, when the caller
+// gives no status array, their status.  A context keeps a few sets: the steps
+// of one stream share one, so that steps on up to kLaneScratch streams do not
+// wait for each other.  Steps that share a set are ordered on the device by
+// its event (recorded after a step's last launch, waited for by the next).
+constexpr int kLaneScratch = 4;  // the device's hardware queues
+struct LaneScratch {
+  int32_t* esc_list = nullptr;  // the number of cells handed over (64 bits, kEscHeader ints),
+                                // then the cells
+  int64_t esc_cap = 0;
+  int32_t* status = nullptr;
+  int64_t status_cap = 0;
+  hipEvent_t done = nullptr;
+  bool used = false;
+  hipStream_t stream = nullptr;  // of its last step
+};
+
 struct pfchem_ctx {
   int device = 0;
   int num_cus = 256;
@@ -40,14 +57,12 @@ struct pfchem_ctx {
   LaunchCfg vlaunch[2][kBuckets];
   int32_t* buckets = nullptr;  // kBuckets lists of ncell entries, then the counts
   int64_t bucket_cap = 0;
-  int32_t* esc_list = nullptr;  // the number of cells the one-lane pass handed over (64 bits,
-                                // kEscHeader ints), then the cells
-  int64_t esc_cap = 0;
-  // steps that use the scratch lists held here (escalated cells, status
-  // scratch, size buckets) are ordered on the device: each records this
-  // event after its last launch and the next one's stream waits for it
+  // steps that use the size buckets are ordered on the device: each records
+  // this event after its last launch and the next one's stream waits for it
   hipEvent_t scratch_done = nullptr;
   bool scratch_done_used = false;
+  LaneScratch lane_scratch[kLaneScratch];
+  int lane_scratch_next = 0;
   // pfchem_set_pass_timing: events around the one-lane pass of a step
   bool pass_timing = false;
   bool pass_recorded = false;
@@ -88,8 +103,6 @@ struct pfchem_ctx {
   std::string lane_adj_src;  // the adjoint module's source (compiled at first use)
   bool lane_adj_ready = false;
   LaunchCfg team_default{16, 1, 256, 4};  // team shape of the FP64 rescue pass
-  int32_t* status_scratch = nullptr;      // per-cell status when the caller gives none
-  int64_t status_cap = 0;
   // launch-shape cache identity: device architecture and a hash of the
   // network arrays and options
   std::string arch = "gfx";
@@ -165,11 +178,11 @@ unsigned long long* slot_cursors(pfchem_ctx* ctx, int k) {
   return ctx->counter + (size_t)k * kCursorWords;
 }
 
-// before a scratch list is freed / regrown: every step that used it is done
+// before the bucket lists are freed / regrown: every step that used them is done
 void scratch_quiesce(pfchem_ctx* ctx) {
   if (ctx->scratch_done_used) (void)hipEventSynchronize(ctx->scratch_done);
 }
-// a step that uses the scratch lists starts after the previous such step
+// a step that uses the bucket lists starts after the previous such step
 hipError_t scratch_order(pfchem_ctx* ctx, hipStream_t s) {
   return ctx->scratch_done_used ? hipStreamWaitEvent(s, ctx->scratch_done, 0) : hipSuccess;
 }
@@ -177,6 +190,33 @@ hipError_t scratch_release(pfchem_ctx* ctx, hipStream_t s) {
   hipError_t e = hipEventRecord(ctx->scratch_done, s);
   if (e == hipSuccess) ctx->scratch_done_used = true;
   return e;
+}
+
+// the set a one-lane step on `s` uses: its stream's, else one never used, else
+// the next in turn (a captured step takes the first, whose event, once
+// recorded outside the capture, makes the runtime refuse it: a graph must not
+// hold lists that a later step may regrow)
+LaneScratch& lane_scratch(pfchem_ctx* ctx, hipStream_t s, bool captured) {
+  LaneScratch* set = ctx->lane_scratch;
+  if (captured) return set[0];
+  for (int k = 0; k < kLaneScratch; ++k)
+    if (set[k].used && set[k].stream == s) return set[k];
+  for (int k = 0; k < kLaneScratch; ++k)
+    if (!set[k].used) return set[k];
+  const int k = ctx->lane_scratch_next;
+  ctx->lane_scratch_next = (k + 1) % kLaneScratch;
+  return set[k];
+}
+// room for `n` ints in a list of the set; steps that used it are done first
+bool lane_scratch_grow(LaneScratch& set, int32_t*& list, int64_t& cap, int64_t ncell, size_t n) {
+  if (ncell <= cap) return true;
+  if (set.used) (void)hipEventSynchronize(set.done);
+  if (list) (void)hipFree(list);
+  list = nullptr;
+  cap = 0;
+  if (hipMalloc(&list, sizeof(int32_t) * n) != hipSuccess) return false;
+  cap = ncell;
+  return true;
 }
 
 DevState* acquire_slot(pfchem_ctx* ctx, const DevState& d, hipStream_t s, int* idx,
@@ -752,7 +792,10 @@ int pfchem_create(const pfchem_network* net, const pfchem_options* opt, int devi
       pfchem_destroy(ctx);
       return PFCHEM_ERR_HIP;
     }
-  if (hipEventCreateWithFlags(&ctx->scratch_done, hipEventDisableTiming) != hipSuccess) {
+  hipError_t ee = hipEventCreateWithFlags(&ctx->scratch_done, hipEventDisableTiming);
+  for (LaneScratch& set : ctx->lane_scratch)
+    if (ee == hipSuccess) ee = hipEventCreateWithFlags(&set.done, hipEventDisableTiming);
+  if (ee != hipSuccess) {
     pfchem_destroy(ctx);
     return PFCHEM_ERR_HIP;
   }
@@ -845,7 +888,6 @@ int pfchem_destroy(pfchem_ctx* ctx) {
   if (ctx->counter) (void)hipFree(ctx->counter);
   if (ctx->stage) (void)hipFree(ctx->stage);
   if (ctx->buckets) (void)hipFree(ctx->buckets);
-  if (ctx->esc_list) (void)hipFree(ctx->esc_list);
   if (ctx->dnet_dev) (void)hipFree(ctx->dnet_dev);
   if (ctx->dstate_ring) (void)hipFree(ctx->dstate_ring);
   if (ctx->hstate_ring) (void)hipHostFree(ctx->hstate_ring);
@@ -856,11 +898,15 @@ int pfchem_destroy(pfchem_ctx* ctx) {
   if (ctx->sens_copied) (void)hipEventDestroy(ctx->sens_copied);
   if (ctx->sens_work) (void)hipFree(ctx->sens_work);
   if (ctx->con_buf) (void)hipFree(ctx->con_buf);
-  if (ctx->status_scratch) (void)hipFree(ctx->status_scratch);
   if (ctx->tplan) transport_plan_free(ctx->tplan);
   for (int k = 0; k < kStateRing; ++k)
     if (ctx->ring_done[k]) (void)hipEventDestroy(ctx->ring_done[k]);
   if (ctx->scratch_done) (void)hipEventDestroy(ctx->scratch_done);
+  for (LaneScratch& set : ctx->lane_scratch) {
+    if (set.esc_list) (void)hipFree(set.esc_list);
+    if (set.status) (void)hipFree(set.status);
+    if (set.done) (void)hipEventDestroy(set.done);
+  }
   if (ctx->pass_t0) (void)hipEventDestroy(ctx->pass_t0);
   if (ctx->pass_t1) (void)hipEventDestroy(ctx->pass_t1);
   delete ctx;
@@ -949,18 +995,12 @@ static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double d
     if (rc) return fail(ctx, rc, msg);
     ctx->lane_ready = true;
   }
+  LaneScratch& set = lane_scratch(ctx, s, capturing(s));
   int32_t* st = d.status;
   if (!st) {
-    if (ncell > ctx->status_cap) {
-      scratch_quiesce(ctx);
-      if (ctx->status_scratch) (void)hipFree(ctx->status_scratch);
-      ctx->status_scratch = nullptr;
-      ctx->status_cap = 0;
-      if (hipMalloc(&ctx->status_scratch, sizeof(int32_t) * (size_t)ncell) != hipSuccess)
-        return fail(ctx, PFCHEM_ERR_NOMEM, "status scratch");
-      ctx->status_cap = ncell;
-    }
-    st = ctx->status_scratch;
+    if (!lane_scratch_grow(set, set.status, set.status_cap, ncell, (size_t)ncell))
+      return fail(ctx, PFCHEM_ERR_NOMEM, "status scratch");
+    st = set.status;
   }
   LaneArgs a{};
   a.ld = d.ld;
@@ -1000,27 +1040,20 @@ static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double d
   dr.status = st;
   const bool listed = ncell <= 0x7fffffff;
   if (listed) {
-    if (ncell > ctx->esc_cap) {
-      scratch_quiesce(ctx);
-      if (ctx->esc_list) (void)hipFree(ctx->esc_list);
-      ctx->esc_list = nullptr;
-      ctx->esc_cap = 0;
-      if (hipMalloc(&ctx->esc_list, sizeof(int32_t) * ((size_t)ncell + kEscHeader)) != hipSuccess)
-        return fail(ctx, PFCHEM_ERR_NOMEM, "escalated-cell list");
-      ctx->esc_cap = ncell;
-    }
-    a.esc_count = (unsigned long long*)ctx->esc_list;
-    a.esc_list = ctx->esc_list + kEscHeader;
+    if (!lane_scratch_grow(set, set.esc_list, set.esc_cap, ncell, (size_t)ncell + kEscHeader))
+      return fail(ctx, PFCHEM_ERR_NOMEM, "escalated-cell list");
+    a.esc_count = (unsigned long long*)set.esc_list;
+    a.esc_list = set.esc_list + kEscHeader;
     dr.cell_list = a.esc_list;
-    dr.list_count = ctx->esc_list;  // the low word of the count (< 2^31)
+    dr.list_count = set.esc_list;  // the low word of the count (< 2^31)
   }
   // one descriptor slot (and its cursors) for both launches of this step
   int k = 0;
   DevState* slot = acquire_slot(ctx, dr, s, &k, &e);
   if (e != hipSuccess) return hip_fail(ctx, e, "state descriptor copy");
   unsigned long long* cursors = slot_cursors(ctx, k);
-  // a step on another stream may still use the list / status scratch
-  e = scratch_order(ctx, s);
+  // an earlier step may still use the set
+  if (set.used) e = hipStreamWaitEvent(s, set.done, 0);
   if (e == hipSuccess && ctx->pass_timing) e = hipEventRecord(ctx->pass_t0, s);
   if (e == hipSuccess)
     e = lane_launch(ctx->lane_src, ctx->device, mixed ? 1 : 0, a, ctx->num_cus, bpc, cursors,
@@ -1040,7 +1073,7 @@ static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double d
     LaneArgs b = a;
     b.rescue = 1;
     b.list = a.esc_list;
-    b.list_count = ctx->esc_list;
+    b.list_count = set.esc_list;
     b.esc_list = nullptr;
     b.list_min = ctx->lane_ok && ctx->net.naqcomp < kProdMinAq ? kLaneListMin : 0;
     e = lane_launch(ctx->lane_src, ctx->device, 0, b, ctx->num_cus,
@@ -1052,7 +1085,11 @@ static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double d
                        ctx->team_default, cursors + 32 * ctx->nxcd, ctx->num_cus, ctx->nxcd, s,
                        true);
   if (e == hipSuccess) e = release_slot(ctx, k, s);
-  if (e == hipSuccess) e = scratch_release(ctx, s);
+  if (e == hipSuccess) e = hipEventRecord(set.done, s);
+  if (e == hipSuccess) {
+    set.used = true;
+    set.stream = s;
+  }
   if (e != hipSuccess) return hip_fail(ctx, e, "team rescue launch");
   return PFCHEM_OK;
 }
