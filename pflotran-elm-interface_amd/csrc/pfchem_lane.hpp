@@ -1315,7 +1315,8 @@ __device__ __forceinline__ void lane_step(const Args& A) {
           // dry cells: RReaction adds nothing (reaction.F90:4083)
           const double Rm = r.Im * vol * wm;
           // d res / d ln m_j = nu_i (dIm/dQK QK V rho/1000) nu_j, in units of jc
-          const double gm = r.dIm * vol * QK * dkl * ijc;
+          // (an inactive mineral's Q/K may be infinite)
+          const double gm = r.active ? r.dIm * vol * QK * dkl * ijc : 0.0;
           sfor<0, ns>([&](auto Q) {
             constexpr int a = decltype(Q)::value;
             constexpr int ia = Net::MNRL_ID[mi][a];

@@ -77,3 +77,23 @@ def test_activities_out_of_product_range(tmp_path):
     wl.state = st.subset(np.flatnonzero(ok))
     assert np.all(wl.state["pri_molal"][j] < 1e-58)
     _compare(_reseat(wl), tmp_path, False)
+
+
+@pytest.mark.parametrize("naq", [8, 9])
+def test_inactive_mineral_with_overflowing_saturation(naq, tmp_path, monkeypatch):
+    """a mineral without surface area takes no part, also where its Q/K leaves
+    the FP64 range: the step is the one with a small Q/K, bit for bit, and no
+    further cell is handed over (FP32 pass alone and FP64)"""
+    wl = workloads.random_network_workload(ncell=64, naq=naq, ncplx=16, nmnrl=3, seed=20261213)
+    wl.state["mnrl_area"][1, :] = 0.0
+    monkeypatch.setenv("PFCHEM_HOST_NO_RESCUE", "1")
+    out = []
+    for logk in (0.0, -400.0):  # Q/K = Q 1e400
+        wl.net.kinmnrl_logK[1] = logk
+        exe = LU.build_host(wl.net, wl.opt, str(tmp_path))
+        out.append([LU.run_host(exe, wl.state, wl.dt, f32=f32) for f32 in (False, True)])
+    for small, large in zip(*out):
+        assert (small["status"][0] == 0).mean() > 0.9
+        for f in ("status", "num_iterations", "pri_molal", "total", "sec_molal", "mnrl_volfrac",
+                  "mnrl_rate"):
+            assert np.array_equal(small[f], large[f]), f
