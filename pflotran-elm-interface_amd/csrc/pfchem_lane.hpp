@@ -1448,7 +1448,7 @@ __device__ __forceinline__ void lane_step(const Args& A) {
         // where it starts empty.
         const double av = (double)(pv < (JT)0 ? -pv : pv);
         constexpr bool below = lu_eliminates(p);
-        if (!(av > (below ? kLuTol * amax[p] : 0.0) && av - av == 0.0)) bad = true;  // or not finite
+        if (!(av > (below ? kLuTol * amax[p] : 0.0) && av < 1.0e300)) bad = true;  // or not finite
         const JT inv = F32 ? (JT)1 / pv : (JT)rcp_nr((double)pv);
         pinv[p] = inv;
         sfor<p + 1, N>([&](auto Q) {
