@@ -1306,7 +1306,7 @@ __device__ __forceinline__ void lane_step(const Args& A) {
           const double aff = 1.0 - QK;
           r.active = ar != 0.0 && (PF_VF(mi) > 0.0 || QK > 1.0);
           r.Im = r.active ? -(ar * aff) * Net::MNRL_K[mi] : 0.0;
-          r.dIm = r.active ? ar * Net::MNRL_K[mi] : 0.0;
+          r.dIm = ar * Net::MNRL_K[mi];
         } else {
           r = mineral_rate<mi>(QK, PF_VF(mi), ar, temp);
         }
@@ -1315,7 +1315,7 @@ __device__ __forceinline__ void lane_step(const Args& A) {
           // dry cells: RReaction adds nothing (reaction.F90:4083)
           const double Rm = r.Im * vol * wm;
           // d res / d ln m_j = nu_i (dIm/dQK QK V rho/1000) nu_j, in units of jc
-          // (an inactive mineral's Q/K may be infinite)
+          // (selected here: an inactive mineral's Q/K may be infinite)
           const double gm = r.active ? r.dIm * vol * QK * dkl * ijc : 0.0;
           sfor<0, ns>([&](auto Q) {
             constexpr int a = decltype(Q)::value;
