@@ -1075,7 +1075,7 @@ static int lane_step(pfchem_ctx* ctx, int64_t ncell, const DevState& d, double d
     b.list = a.esc_list;
     b.list_count = set.esc_list;
     b.esc_list = nullptr;
-    b.list_min = ctx->lane_ok && ctx->net.naqcomp < kProdMinAq ? kLaneListMin : 0;
+    b.list_min = ctx->net.naqcomp < kProdMinAq ? kLaneListMin : 0;
     e = lane_launch(ctx->lane_src, ctx->device, 0, b, ctx->num_cus,
                     l64.lanes_per_cell == 1 ? l64.blocks_per_cu : 0, cursors + 16 * ctx->nxcd, 0, s);
     if (e != hipSuccess) return hip_fail(ctx, e, "lane kernel launch (FP64 list)");

@@ -37,10 +37,15 @@
 //     untouched, to a later pass: status kEscalate.
 // With packed FP32 off, FP32 and FP64 instructions issue at the same rate on
 // gfx950, and forming an FP32 entry takes three instructions (multiply,
-// convert, FMA) where an FP64 one takes an FMA: the FP32 pass saves registers
-// only.  Where the FP32 Newton iteration ends is decided by the rounding of
-// its factorization in one cell of a hundred, so its arithmetic is left as it
-// is rather than moved to FP64 accumulation or another scaling.
+// convert, FMA) where an FP64 one takes an FMA.  What FP32 saves is registers,
+// and only where the system is what fills them: the SomDec step takes 256
+// VGPRs + 129 AGPRs against 256 + 222, the step of 15 primaries and 60
+// complexes 256 + 160 against 256 + 158, neither with scratch.  There the FP32
+// pass also hands over more cells (its pivot test is 1e-6), and the FP64
+// kernel is the faster one.  Where the FP32 Newton iteration ends is decided
+// by the rounding of its factorization in one cell of a hundred, so its
+// arithmetic is left as it is rather than moved to FP64 accumulation or
+// another scaling.
 #pragma once
 
 namespace pflane {

@@ -111,3 +111,27 @@ def test_tuning_keeps_the_one_lane_step(variant, tmp_path):
     other = Context(wl.net, wl.opt)
     other.autotune(ds, wl.dt, variant, cache_path=cache)  # the cached choice
     assert _one_lane(other, small, variant)
+
+
+@pytest.mark.parametrize("which", ["inhibition", "pool-monod", "responses", "scalars",
+                                   "no-smoothing", "trackers"])
+def test_somdec_options_on_the_device(which):
+    """networks that reach the sandbox's other options, through the device
+    build of the kernel and its hand-over (test_lane_host_somdec.py runs every
+    option through the host build): the oracle's band on the cells that take
+    its sub-steps, which all but a few do"""
+    import somdec_util as SU
+    wl = SU.option_workload(which, 2049)
+    n = wl.state.ncell
+    ref, rec, nfail = G.run_oracle(wl)
+    assert nfail == 0
+    band = _oracle_band(wl, ref)
+    for variant in VARIANTS:
+        print("case", which, abi.KERNEL_NAMES[variant], flush=True)
+        got, ctx = G.run_gpu(wl, variant)
+        assert np.all(got["status"] == 0)
+        same = got["num_sub_steps"][0] == ref["num_sub_steps"][0]
+        assert (~same).sum() <= max(2, n // 1000)
+        for f in FIELDS:
+            err = np.abs(got[f] - ref[f])
+            assert not (err > 1e-8 * np.abs(ref[f]) + band[f])[:, same].any(), f
