@@ -387,7 +387,9 @@ int pfchem_residual(pfchem_ctx* ctx, int64_t ncell, const pfchem_state* state,
    jac may be NULL.  Replaces the per-cell loop bodies of RTResidualNonFlux
    (reactive_transport.F90:2393-2430, 2599-2642) and RTJacobianNonFlux
    (:3172-3183, 3270-3300) for a batch of cells.  The first call of a network
-   that the one-lane kernel takes compiles its module. */
+   of up to 160 complexes that the one-lane kernel takes compiles its module;
+   the team kernel runs the others, a first call inside a stream capture, and
+   a network whose module does not compile. */
 int pfchem_residual_jacobian(pfchem_ctx* ctx, int64_t ncell, const pfchem_state* state,
                              const double* fixed_total, const double* fixed_immobile,
                              double dt, double* res, double* jac, void* stream);
