@@ -11,8 +11,8 @@ import lane_util as LU
 from test_gpu_residual import DT, _case, _oracle
 
 
-@pytest.mark.parametrize("which", ["calcite", "random15"])
-@pytest.mark.parametrize("act_h2o", [False, True])
+@pytest.mark.parametrize("which,act_h2o", [("calcite", False), ("calcite", True),
+                                           ("random15", False)])
 def test_residual_reads_the_water_activity(which, act_h2o, tmp_path):
     wl, st, fixed, fimm = _case(which, 65)
     n, net = st.ncell, wl.net
