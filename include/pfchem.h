@@ -401,7 +401,8 @@ int pfchem_residual_jacobian(pfchem_ctx* ctx, int64_t ncell, const pfchem_state*
    16 primaries (plus immobile species with first-order decay) without the
    SomDec sandbox or per-cell active counts, and is then the default.
    A SomDec network without complexes, minerals, an oxygen response and O2
-   tracking runs it by default too.  The launch reported for that default is
+   tracking, of at most 288 Jacobian entries (fill-in of its elimination
+   included; the ELM-CN cascade has 115), runs it by default too.  The launch reported for that default is
    the team shape of the cells the kernel hands over, and setting that shape
    restores the default; any other team shape runs the team kernel alone.
    block_size must be 256 and blocks_per_cu caps the workgroups per CU (0:
